@@ -17,6 +17,23 @@ typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
 namespace fni8 {
 
+// 16 bytes at a 4-byte aligned address (one global_load_dwordx4 either way).
+typedef i32x4 i32x4_a4 __attribute__((aligned(4)));
+
+// Bytes k .. k+15 of a 4-byte aligned row of K (a multiple of 4) bytes; zeros
+// past the row's end, which is never read.
+__device__ __forceinline__ i32x4 ld16_tail(const int8_t* row, int64_t k, int K) {
+    i32x4 v = {0, 0, 0, 0};
+    if (k + 16 <= K) {
+        v = *reinterpret_cast<const i32x4_a4*>(row + k);
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            if (k + 4 * t < K) v[t] = *reinterpret_cast<const int32_t*>(row + k + 4 * t);
+    }
+    return v;
+}
+
 // 16x16x64 int8 MFMA (CDNA4).  srcA lane l carries 16 int8 of row (l % 16),
 // srcB lane l carries 16 int8 of column (l % 16); both use the same k subset,
 // chosen by (l / 16).  Result lane l, register r holds D[4*(l/16) + r][l % 16].

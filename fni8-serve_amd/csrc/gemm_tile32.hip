@@ -26,7 +26,9 @@ using fni8t::i32x16;
 using fni8t::dense_tile;
 using fni8t::tile_epilogue;
 
+template <bool ALIGNED4>
 __device__ __forceinline__ i32x4 ld16(const int8_t* p) {
+    if constexpr (ALIGNED4) return *reinterpret_cast<const fni8::i32x4_a4*>(p);
     return *reinterpret_cast<const i32x4*>(p);
 }
 
@@ -37,7 +39,11 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int BM, int BN, int BK, bool GROUPED, bool WRITE_ACC>
+// RAGGED: any K that is a multiple of 4 and rows that are only 4-byte aligned.
+// The K steps are rounded up to an even number; a step that reaches past K
+// takes its chunks through ld16_tail (zeros past the row's end on both sides,
+// so the products there vanish), every other step runs the same loads.
+template <int BM, int BN, int BK, bool GROUPED, bool WRITE_ACC, bool RAGGED>
 __global__ __launch_bounds__(512) void gemm_tile32_kernel(
     const int8_t* __restrict__ aq, int64_t lda, const float* __restrict__ as,
     const int32_t* __restrict__ row_index, int M, int K, const int8_t* __restrict__ w,
@@ -51,6 +57,7 @@ __global__ __launch_bounds__(512) void gemm_tile32_kernel(
     constexpr int FM = WTM / 32, FN = WTN / 32;
     constexpr int A_CH = BM * CPR / NT, B_CH = BN * CPR / NT;
     static_assert(A_CH * NT == BM * CPR && B_CH * NT == BN * CPR, "tile/threads mismatch");
+    static_assert(NT % CPR == 0, "a thread keeps one chunk column");
     constexpr int BUF = (BM + BN) * LDSR;
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
 
@@ -102,10 +109,20 @@ __global__ __launch_bounds__(512) void gemm_tile32_kernel(
     auto gload = [&](int kt, auto slot_c) {
         constexpr int slot = decltype(slot_c)::value;
         const int64_t ko = (int64_t)kt * BK;
+        if constexpr (RAGGED) {
+            if (ko + BK > K) {
+                const int c = (tid % CPR) * 16;  // every chunk of a thread has this offset
 #pragma unroll
-        for (int i = 0; i < A_CH; i++) ra[slot][i] = ld16(asrc[i] + ko);
+                for (int i = 0; i < A_CH; i++) ra[slot][i] = fni8::ld16_tail(asrc[i] - c, ko + c, K);
 #pragma unroll
-        for (int i = 0; i < B_CH; i++) rb[slot][i] = ld16(bsrc[i] + ko);
+                for (int i = 0; i < B_CH; i++) rb[slot][i] = fni8::ld16_tail(bsrc[i] - c, ko + c, K);
+                return;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < A_CH; i++) ra[slot][i] = ld16<RAGGED>(asrc[i] + ko);
+#pragma unroll
+        for (int i = 0; i < B_CH; i++) rb[slot][i] = ld16<RAGGED>(bsrc[i] + ko);
     };
     auto sstore = [&](auto buf_c, auto slot_c) {
         constexpr int buf = decltype(buf_c)::value, slot = decltype(slot_c)::value;
@@ -161,7 +178,8 @@ __global__ __launch_bounds__(512) void gemm_tile32_kernel(
 
     using C0 = std::integral_constant<int, 0>;
     using C1 = std::integral_constant<int, 1>;
-    const int KT = K / BK;  // even and >= 2 (checked by the launcher)
+    // even and >= 2 (for whole steps checked by the launcher)
+    const int KT = RAGGED ? ((K - 1) / (2 * BK) + 1) * 2 : K / BK;
     // Every variant runs the same loads, LDS stores and barriers; only the
     // MFMA work differs.
     auto mainloop = [&](auto live_c) {
@@ -205,7 +223,7 @@ __global__ __launch_bounds__(512) void gemm_tile32_kernel(
                                              n0, N, bexp != nullptr, y, ldy, acc_out);
 }
 
-template <int BM, int BN, int BK, bool GROUPED>
+template <int BM, int BN, int BK, bool GROUPED, bool RAGGED = false>
 int launch(const int8_t* aq, int64_t lda, const float* as, const int32_t* row_index, int M,
            int K, const int8_t* w, const float* ws, int N, int E, const int32_t* seg_off,
            const uint16_t* bias, uint16_t* y, int64_t ldy, int32_t* acc_out, unsigned slots,
@@ -222,7 +240,7 @@ int launch(const int8_t* aq, int64_t lda, const float* as, const int32_t* row_in
     // again with the same value is idempotent, so a race between threads is harmless.
     auto run = [&](auto acc_c) -> int {
         constexpr bool ACC = decltype(acc_c)::value;
-        const auto kern = gemm_tile32_kernel<BM, BN, BK, GROUPED, ACC>;
+        const auto kern = gemm_tile32_kernel<BM, BN, BK, GROUPED, ACC, RAGGED>;
         static bool attr_set = false;
         if (!attr_set) {
             hipError_t e = hipFuncSetAttribute((const void*)kern,
@@ -245,25 +263,37 @@ int launch(const int8_t* aq, int64_t lda, const float* as, const int32_t* row_in
 
 namespace fni8h {
 
-// Returns 1 if the shape was not taken (the caller falls back), else an FNI8 code.
+// Takes every shape: K steps of 128 (or 64) bytes and an even number of them
+// where the operands are 16-byte aligned, and the ragged form of the 128-byte
+// steps for everything else.  Measured on MI355X, M = 777 (us, before -> with the
+// ragged form): N x K = 4096 x 1376 2327 -> 14.0 and 3130 x 2080 4731 -> 23.8
+// (before: one dot4 output per lane), 4096 x 2112 29.9 -> 18.1 and 4096 x 1088
+// 22.4 -> 12.4 (before: 16x16x64 MFMA tiles, half the int8 rate).
 int launch_tile32(const int8_t* aq, int64_t lda, const float* as, const int32_t* row_index,
                   int64_t M, int64_t K, const int8_t* w, const float* ws, int64_t N, int64_t E,
                   const int32_t* seg_off, const uint16_t* bias, uint16_t* y, int64_t ldy,
                   int32_t* acc_out, hipStream_t st) {
-    // K steps of 128 (or 64) bytes, an even number of them
-    const bool k128 = K % 256 == 0, k64 = !k128 && K % 128 == 0;
-    if (!(k128 || k64)) return 1;
+    const bool al16 = lda % 16 == 0 && (uintptr_t)aq % 16 == 0 && (uintptr_t)w % 16 == 0;
+    const bool k128 = al16 && K % 256 == 0, k64 = al16 && K % 256 == 128;
+    const bool ragged = !k128 && !k64;
     const int m = (int)M, k = (int)K, n = (int)N, e = (int)E;
     if (E > 0) {
         // Segment tiles by average rows per expert, measured on the 128-expert
         // top-8 MoE projections at T = 32..4096: 64x128 up to 40 rows (less
         // padding in each expert's last tile), 128x128 above (6-14% faster than
         // 128x256 at T = 1024..4096: twice the n-tiles fill the CUs better).
-        if (k128 && (double)M / (double)E <= 40.0)
+        const unsigned slots64 = (unsigned)((M + 63) / 64 + E);
+        const bool few = (double)M / (double)E <= 40.0;
+        if (k128 && few)
             return launch<64, 128, 128, true>(aq, lda, as, row_index, m, k, w, ws, n, e, seg_off,
-                                              bias, y, ldy, acc_out,
-                                              (unsigned)((M + 63) / 64 + E), st);
+                                              bias, y, ldy, acc_out, slots64, st);
+        if (ragged && few)
+            return launch<64, 128, 128, true, true>(aq, lda, as, row_index, m, k, w, ws, n, e,
+                                                    seg_off, bias, y, ldy, acc_out, slots64, st);
         const unsigned slots = (unsigned)((M + 127) / 128 + E);
+        if (ragged)
+            return launch<128, 128, 128, true, true>(aq, lda, as, row_index, m, k, w, ws, n, e,
+                                                     seg_off, bias, y, ldy, acc_out, slots, st);
         if (k128)
             return launch<128, 128, 128, true>(aq, lda, as, row_index, m, k, w, ws, n, e, seg_off,
                                                bias, y, ldy, acc_out, slots, st);
@@ -284,9 +314,10 @@ int launch_tile32(const int8_t* aq, int64_t lda, const float* as, const int32_t*
         return n;
     }();
     constexpr int kTiles[6][2] = {{256, 256}, {128, 256}, {256, 128}, {128, 128}, {64, 256}, {64, 128}};
-    int best = 0;
+    int best = 2;
     double best_fill = -1.0;
     for (int i = 0; i < 6; i++) {
+        if (ragged && (i <= 1 || i == 4)) continue;  // three of them have a ragged form
         const int64_t wgs = ((M + kTiles[i][0] - 1) / kTiles[i][0]) * ((N + kTiles[i][1] - 1) / kTiles[i][1]);
         const double fill = (double)wgs / (double)(((wgs + cus - 1) / cus) * cus);
         if (fill > best_fill + 1e-9) {
@@ -302,6 +333,16 @@ int launch_tile32(const int8_t* aq, int64_t lda, const float* as, const int32_t*
 #define FNI8_T32_K128(BM, BN)                                                                     \
     return launch<BM, BN, 128, false>(aq, lda, as, row_index, m, k, w, ws, n, e, seg_off, bias, y,  \
                                       ldy, acc_out, 0, st)
+    if (ragged) {
+        if (best == 2)
+            return launch<256, 128, 128, false, true>(aq, lda, as, row_index, m, k, w, ws, n, e,
+                                                      seg_off, bias, y, ldy, acc_out, 0, st);
+        if (best == 3)
+            return launch<128, 128, 128, false, true>(aq, lda, as, row_index, m, k, w, ws, n, e,
+                                                      seg_off, bias, y, ldy, acc_out, 0, st);
+        return launch<64, 128, 128, false, true>(aq, lda, as, row_index, m, k, w, ws, n, e,
+                                                 seg_off, bias, y, ldy, acc_out, 0, st);
+    }
     // 64-row tiles need 128-byte K steps (one 16-byte chunk per thread and operand)
     if (!k128 && best >= 4) best = 3;
     switch (best) {
