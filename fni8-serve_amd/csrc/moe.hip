@@ -1,11 +1,13 @@
 // MoE routing sort and weighted combine (gfx950).
 //
-// sort:    one workgroup per expert.  Pass 1 counts ids below and equal to the
-//          expert (block reduction) -> the segment start, with no global
-//          atomics.  Pass 2 walks the T*k ids in order and places the expert's
-//          entries with a block-wide exclusive scan, so the segment keeps the
+// sort:    one workgroup per expert, its waves owning contiguous runs of the T*k
+//          ids.  Pass 1 counts the ids below and equal to the expert (one block
+//          exchange) -> the segment start and each wave's first row, with no
+//          global atomics.  Pass 2 places the wave's entries in id order (the
+//          rank inside 256 ids from four ballots), so the segment keeps the
 //          (token, slot) order of `(topi == e).nonzero()` -- a deterministic,
-//          stable counting sort.  The ids are read twice per workgroup from L2.
+//          stable counting sort.  Up to 2048 ids a wave stay in registers
+//          between the passes.
 // combine: one workgroup per token; each lane owns 8 consecutive hidden
 //          elements and sums the token's expert rows in ascending expert id
 //          with fp16 rounding after every product and add, matching the
@@ -14,73 +16,103 @@
 
 namespace {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortPer = 4;  // ids per thread per chunk
 constexpr int kMaxTopK = 32;
 
-__device__ __forceinline__ int block_excl_scan(int v, int* lds, int& total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int incl = fni8::wave_incl_scan_i32(v, lane);
-    if (lane == 63) lds[wave] = incl;
-    __syncthreads();
-    int before = 0;
-    total = 0;
-#pragma unroll
-    for (int i = 0; i < kSortThreads / 64; i++) {
-        const int t = lds[i];
-        before += i < wave ? t : 0;
-        total += t;
-    }
-    __syncthreads();
-    return before + incl - v;
-}
-
-__global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
+// Bound by latency: every workgroup reads all ids (from L2) and meets once.
+// Walking 1024 ids at a time with two block barriers each took 47 us for 24000
+// ids and 128 experts on MI355X; this takes 9 (16 waves; few ids keep 4 waves,
+// which start sooner).
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void moe_sort_kernel(
     const int32_t* __restrict__ topi, int Tk, int k, int E, int32_t* __restrict__ seg_off,
     int32_t* __restrict__ row_token, int32_t* __restrict__ pos) {
-    __shared__ int lds[kSortThreads / 64];
+    constexpr int STEP = 256;  // ids per wave and step, four per lane
+    constexpr int KEEP = 8;    // steps held in registers
+    __shared__ int lds[2][WAVES];
     const int e = blockIdx.x;
-    const int tid = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int steps = (Tk + STEP * WAVES - 1) / (STEP * WAVES);
+    const int64_t first = (int64_t)wave * steps * STEP + lane * 4;
 
-    int lt = 0, eq = 0;
-    for (int i = tid; i < Tk; i += kSortThreads) {
-        const int id = topi[i];
-        lt += (id >= 0 && id < e) ? 1 : 0;
-        eq += id == e ? 1 : 0;
-    }
-    int tot_lt, tot_eq;
-    block_excl_scan(lt, lds, tot_lt);
-    block_excl_scan(eq, lds, tot_eq);
-    if (tid == 0) {
-        seg_off[e] = tot_lt;
-        if (e == E - 1) seg_off[E] = tot_lt + tot_eq;
-    }
-
-    int base = tot_lt;
-    for (int c0 = 0; c0 < Tk; c0 += kSortThreads * kSortPer) {
-        const int i0 = c0 + tid * kSortPer;
-        bool hit[kSortPer];
-        int cnt = 0;
+    // ids i .. i+3 (-1 past the end)
+    auto load = [&](int s) {
+        const int64_t i = first + (int64_t)s * STEP;
+        i32x4 v = {-1, -1, -1, -1};
+        if (i + 3 < Tk) {
+            v = *reinterpret_cast<const fni8::i32x4_a4*>(topi + i);
+        } else {
 #pragma unroll
-        for (int j = 0; j < kSortPer; j++) {
-            hit[j] = (i0 + j < Tk) && topi[i0 + j] == e;
-            cnt += hit[j] ? 1 : 0;
+            for (int j = 0; j < 4; j++)
+                if (i + j < Tk) v[j] = topi[i + j];
         }
-        int chunk_total;
-        int p = base + block_excl_scan(cnt, lds, chunk_total);
+        return v;
+    };
+    int lt = 0, eq = 0;
+    auto count = [&](i32x4 v) {
 #pragma unroll
-        for (int j = 0; j < kSortPer; j++) {
-            if (hit[j]) {
-                row_token[p] = (i0 + j) / k;
-                pos[i0 + j] = p;
+        for (int j = 0; j < 4; j++) {
+            lt += (v[j] >= 0 && v[j] < e) ? 1 : 0;
+            eq += v[j] == e ? 1 : 0;
+        }
+    };
+    i32x4 kept[KEEP];
+#pragma unroll
+    for (int s = 0; s < KEEP; s++) kept[s] = s < steps ? load(s) : i32x4{-1, -1, -1, -1};
+#pragma unroll
+    for (int s = 0; s < KEEP; s++) count(kept[s]);
+    for (int s = KEEP; s < steps; s++) count(load(s));
+    lt = fni8::wave_sum_i32(lt);
+    eq = fni8::wave_sum_i32(eq);
+    if (lane == 0) {
+        lds[0][wave] = lt;
+        lds[1][wave] = eq;
+    }
+    __syncthreads();
+    int start = 0, total = 0, before = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+        start += lds[0][w];
+        total += lds[1][w];
+        before += w < wave ? lds[1][w] : 0;
+    }
+    if (threadIdx.x == 0) {
+        seg_off[e] = start;
+        if (e == E - 1) seg_off[E] = start + total;
+    }
+
+    int base = start + before;
+    const uint64_t below = ((uint64_t)1 << lane) - 1;  // the lanes before this one
+    auto place = [&](i32x4 v, int s) {
+        const int64_t i = first + (int64_t)s * STEP;
+        if (e == 0) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (i + j < Tk && (v[j] < 0 || v[j] >= E)) pos[i + j] = -1;  // no row
+        }
+        uint64_t hit[4];
+        int p = base, n = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            hit[j] = __ballot(v[j] == e);
+            p += __builtin_popcountll(hit[j] & below);
+            n += __builtin_popcountll(hit[j]);
+        }
+        if (n == 0) return;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (v[j] == e) {
+                row_token[p] = (int)((uint32_t)(i + j) / (uint32_t)k);
+                pos[i + j] = p;
                 p++;
-            } else if (e == 0 && i0 + j < Tk) {
-                const int id = topi[i0 + j];
-                if (id < 0 || id >= E) pos[i0 + j] = -1;  // out-of-range id: no row
             }
         }
-        base += chunk_total;
-    }
+        base += n;
+    };
+#pragma unroll
+    for (int s = 0; s < KEEP; s++)
+        if (s < steps) place(kept[s], s);
+    for (int s = KEEP; s < steps; s++) place(load(s), s);
 }
 
 // Combine for k <= KM (the common top-8): the slots are sorted by expert id
@@ -224,8 +256,13 @@ namespace fni8h {
 
 int launch_moe_sort(const int32_t* topi, int64_t T, int64_t k, int64_t E, int32_t* seg_off,
                     int32_t* row_token, int32_t* pos, hipStream_t st) {
-    hipLaunchKernelGGL(moe_sort_kernel, dim3((unsigned)E), dim3(kSortThreads), 0, st, topi,
-                       (int)(T * k), (int)k, (int)E, seg_off, row_token, pos);
+    // 4 waves hold 2048 ids in two steps each; above, 16 waves
+    if (T * k <= 2048)
+        hipLaunchKernelGGL(moe_sort_kernel<4>, dim3((unsigned)E), dim3(4 * 64), 0, st, topi,
+                           (int)(T * k), (int)k, (int)E, seg_off, row_token, pos);
+    else
+        hipLaunchKernelGGL(moe_sort_kernel<16>, dim3((unsigned)E), dim3(16 * 64), 0, st, topi,
+                           (int)(T * k), (int)k, (int)E, seg_off, row_token, pos);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error_detail("moe_sort launch: %s", hipGetErrorString(e));
