@@ -17,6 +17,9 @@
 // product does not care in which order its terms come.  Sign extension of a
 // nibble u in each byte is ((u ^ 8) + 0x78) ^ 0x80: the sum stays below 0x88,
 // so no carry crosses a byte.
+#include <type_traits>
+
+#include "tile_common.h"
 #include "w4a8_common.h"
 
 namespace {
@@ -594,50 +597,75 @@ __global__ __launch_bounds__(WAVES * 64) void w4a8_mfma_kernel(
 
 // ---- prefill: MFMA tile, group-wise fp32 fold --------------------------------
 //
-// Workgroup of 4 waves (2 x 2) over a BM x BN tile; each wave a (BM/2) x (BN/2)
-// block of 32x32 accumulators.  K is consumed in steps of KS = min(G, 128)
-// codes: the activation step (split into even / odd k) and the unpacked weight
-// step go to LDS and the 32x32x32 int8 MFMAs add them into int32
-// accumulators; after the last step of a group every accumulator is folded
-// into its fp32 sum with the group scale of its column and reset.  The next
-// step's global loads are in flight during the current step's MFMAs.
+// Workgroup of 4 waves (2 x 2) over a 128 x 128 tile; each wave a 64 x 64 block,
+// as 2 x 2 blocks of 32x32.  K is consumed in steps of KS codes through two LDS
+// stages with one barrier a step: the next step's global loads are in flight
+// during the current step and go to the other stage at its end.  The packed
+// weights are unpacked on the way to LDS, each nibble into the high half of its
+// byte (16 * code, natural k order), so the activations are stored unchanged.
+//
+// The fold of every accumulator with its group scale is what bounds this kernel:
+// a conversion and an FMA per output element and group are as many VALU cycles as
+// the group's MFMAs take at 128 codes.  So the two run side by side in each wave:
+// while the MFMAs of one 32-row half of the wave's block write their int32 sums,
+// the other half's finished sums are folded.  Only the sums of the current group
+// exist (each group's first MFMA adds to an inline zero), and two waves a SIMD
+// fit in 256 registers each, so the sums stay in registers that the VALU reads
+// directly; with all of them held across a step in the accumulation registers,
+// every sum cost a third instruction to move.
+//
+// The sums are 16 * acc_g, and the running sums hold 16 times the fold's value:
+// fma((float)(16 acc_g), ws, 16 accf) rounds exactly as fma((float)acc_g, ws, accf)
+// scaled by 16, and the epilogue multiplies by 1/16 first.
+//
 // GROUPED: the expert-segment form (the MoE layer's projections, one launch):
-// blockIdx.x is one BM-row tile of one expert's sorted segment, blockIdx.y the
+// blockIdx.x is one 128-row tile of one expert's sorted segment, blockIdx.y the
 // column tile; sorted row r reads activation row rmap[r] (row r without a map)
 // and its scale; weights, scales and bias are stacked per expert.
-template <int BM, int BN, int G, bool GROUPED = false>
-__global__ __launch_bounds__(256) void w4a8_tile_kernel(
+constexpr int kTileRow = 128 * 2 + 16;  // bytes of a staged output row, padded
+template <int KS>
+constexpr size_t tile_lds() {
+    const size_t stages = (size_t)2 * 256 * (KS + 16);
+    const size_t out = (size_t)128 * kTileRow + 128 * 4;
+    return stages > out ? stages : out;
+}
+
+template <int G, int KS, bool GROUPED = false>
+__global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
     const int8_t* __restrict__ xq, int64_t ldq, const float* __restrict__ xs,
     const int32_t* __restrict__ rmap, int M, int K, const uint8_t* __restrict__ w,
     const float* __restrict__ ws, int N, int E, const int32_t* __restrict__ seg_off,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t ldy) {
-    constexpr int NT = 256;
-    constexpr int KS = G < 128 ? G : 128;   // codes per K-step
-    constexpr int SPG = G / KS;             // steps per group
+    constexpr int BM = 128, BN = 128, NT = 256;
+    constexpr int UK = G < KS ? G : KS;     // codes of one group in a step (a unit)
+    constexpr int UPS = KS / UK;            // units per step
+    constexpr int SPG = G / UK;             // steps per group
+    constexpr int QS = UK / 32;             // MFMAs per block and unit
     constexpr int LDSR = KS + 16;           // padded LDS row (bytes)
-    constexpr int WTM = BM / 2, WTN = BN / 2;
-    constexpr int FM = WTM / 32, FN = WTN / 32;
+    constexpr int STAGE = (BM + BN) * LDSR;
     constexpr int A_TOT = BM * (KS / 16), B_TOT = BN * (KS / 32);  // 16-byte chunks per step
     constexpr int A_CH = (A_TOT + NT - 1) / NT, B_CH = (B_TOT + NT - 1) / NT;
-    __shared__ __attribute__((aligned(16))) int8_t smem[(BM + BN) * LDSR];
+    static_assert(SPG == 1 || (UPS == 1 && SPG == 2), "a step holds whole groups or half of one");
+    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int ng = K / G;
     const int nsteps = K / KS;
     // output rows [m0, mend)
-    int m0 = blockIdx.y * BM, mend = M, n0 = blockIdx.x * BN;
+    int m0, mend, n0;
     if constexpr (GROUPED) {
         // every wave finds the same tile; past the last tile the whole
         // workgroup leaves before any barrier
-        int e, r0, r1;
-        if (!fni8::find_group_tile(seg_off, E, BM, blockIdx.x, M, e, r0, r1)) return;
-        m0 = r0;
-        mend = r1;
+        int e;
+        if (!fni8::find_group_tile(seg_off, E, BM, blockIdx.x, M, e, m0, mend)) return;
         n0 = blockIdx.y * BN;
         w += (int64_t)e * N * (K / 2);
         ws += (int64_t)e * N * ng;
         if (bias != nullptr) bias += (int64_t)e * N;
+    } else {
+        fni8t::dense_tile<BM, BN>(M, N, m0, mend, n0);
     }
     // activation row of output row r
     auto src_row = [&](int r) -> int {
@@ -661,117 +689,214 @@ __global__ __launch_bounds__(256) void w4a8_tile_kernel(
         nr = nr < N ? nr : N - 1;
         bsrc[i] = w + (int64_t)nr * (K / 2) + (c % (KS / 32)) * 16;
     }
-    uint4 ra[A_CH], rb[B_CH];
+    i32x4 ra[A_CH], rb[B_CH];
     auto gload = [&](int s) {
 #pragma unroll
-        for (int i = 0; i < A_CH; i++) ra[i] = *reinterpret_cast<const uint4*>(asrc[i] + (int64_t)s * KS);
+        for (int i = 0; i < A_CH; i++) ra[i] = *reinterpret_cast<const i32x4*>(asrc[i] + (int64_t)s * KS);
 #pragma unroll
         for (int i = 0; i < B_CH; i++)
-            rb[i] = *reinterpret_cast<const uint4*>(bsrc[i] + (int64_t)s * (KS / 2));
+            rb[i] = *reinterpret_cast<const i32x4*>(bsrc[i] + (int64_t)s * (KS / 2));
     };
-    auto sstore = [&]() {
+    auto sstore = [&](int buf) {
+        int8_t* st = smem + buf * STAGE;
 #pragma unroll
         for (int i = 0; i < A_CH; i++) {
             const int c = tid + i * NT;
             if (A_TOT % NT != 0 && c >= A_TOT) continue;
-            uint4 o;
-            split8(ra[i].x, ra[i].y, o.x, o.y);
-            split8(ra[i].z, ra[i].w, o.z, o.w);
-            *reinterpret_cast<uint4*>(smem + (c / (KS / 16)) * LDSR + (c % (KS / 16)) * 16) = o;
+            *reinterpret_cast<i32x4*>(st + (c / (KS / 16)) * LDSR + (c % (KS / 16)) * 16) = ra[i];
         }
 #pragma unroll
         for (int i = 0; i < B_CH; i++) {
             const int c = tid + i * NT;
             if (B_TOT % NT != 0 && c >= B_TOT) continue;
-            uint4 o0, o1;
-            unpack8(rb[i].x, o0.x, o0.y);
-            unpack8(rb[i].y, o0.z, o0.w);
-            unpack8(rb[i].z, o1.x, o1.y);
-            unpack8(rb[i].w, o1.z, o1.w);
-            int8_t* dst = smem + (BM + c / (KS / 32)) * LDSR + (c % (KS / 32)) * 32;
-            *reinterpret_cast<uint4*>(dst) = o0;
-            *reinterpret_cast<uint4*>(dst + 16) = o1;
+            int8_t* dst = st + (BM + c / (KS / 32)) * LDSR + (c % (KS / 32)) * 32;
+            *reinterpret_cast<i32x4*>(dst) = unpack16x16(rb[i][0], rb[i][1]);
+            *reinterpret_cast<i32x4*>(dst + 16) = unpack16x16(rb[i][2], rb[i][3]);
         }
     };
 
-    i32x16 acc[FM][FN];
-    float accf[FM][FN][16];
+    // the group scales of this lane's two columns
+    const float* wsc[2];
 #pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-            acc[i][j] = i32x16{};
-#pragma unroll
-            for (int r = 0; r < 16; r++) accf[i][j][r] = 0.0f;
-        }
-
-    // the group scales of this lane's accumulator columns
-    const float* wsc[FN];
-#pragma unroll
-    for (int j = 0; j < FN; j++) {
-        int n = n0 + wn * WTN + j * 32 + (lane & 31);
+    for (int j = 0; j < 2; j++) {
+        int n = n0 + wn * 64 + j * 32 + (lane & 31);
         n = n < N ? n : N - 1;
         wsc[j] = ws + (int64_t)n * ng;
     }
+    float wnow[UPS][2], wnext[UPS][2];  // scales of the step's units, and of the next group's
+    float wold[2] = {0.0f, 0.0f};  // scales of the sums that half 1 still holds
+    auto wload = [&](int s) {
+#pragma unroll
+        for (int u = 0; u < UPS; u++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) wnext[u][j] = wsc[j][s / SPG * UPS + u];
+    };
+    auto wtake = [&]() {
+#pragma unroll
+        for (int u = 0; u < UPS; u++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) wnow[u][j] = wnext[u][j];
+    };
 
+    i32x16 sum[2][2];        // the group's sums of [half][column block]
+    float accf[2][2][16];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            sum[i][j] = i32x16{};
+#pragma unroll
+            for (int r = 0; r < 16; r++) accf[i][j][r] = 0.0f;
+        }
+    auto fold = [&](auto half_c, const float (&sc)[2]) {
+        constexpr int i = decltype(half_c)::value;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                accf[i][j][r] = __builtin_fmaf((float)sum[i][j][r], sc[j], accf[i][j][r]);
+    };
+    // fragment read: lane l takes row l % 32 of a 32-row block and bytes
+    // 16 * (l / 32) of each 32-byte sub-step (the 32x32x32 operand layout)
     const int fo = (lane & 31) * LDSR + (lane >> 5) * 16;
-    gload(0);
-    for (int s = 0; s < nsteps; s++) {
-        sstore();
-        __syncthreads();
-        if (s + 1 < nsteps) gload(s + 1);
-        const int8_t* ab = smem + (wm * WTM) * LDSR + fo;
-        const int8_t* bb = smem + (BM + wn * WTN) * LDSR + fo;
+    auto products = [&](auto half_c, auto first_c, const i32x4 (&af)[QS], const i32x4 (&bf)[2][QS]) {
+        constexpr int i = decltype(half_c)::value;
 #pragma unroll
-        for (int ks = 0; ks < KS / 32; ks++) {
-            i32x4 af[FM], bf[FN];
+        for (int q = 0; q < QS; q++)
 #pragma unroll
-            for (int i = 0; i < FM; i++)
-                af[i] = *reinterpret_cast<const i32x4*>(ab + i * 32 * LDSR + ks * 32);
+            for (int j = 0; j < 2; j++)
+                sum[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                    af[q], bf[j][q], (decltype(first_c)::value && q == 0) ? i32x16{} : sum[i][j], 0, 0, 0);
+    };
+    using C0 = std::integral_constant<int, 0>;
+    using C1 = std::integral_constant<int, 1>;
+    // One MFMA, then PER VALU instructions, until `products` of one half are
+    // through: keeps the compiler from running all of the one before all of the
+    // other.  The reads of the second half's rows go between.
+    auto interleave = [&](auto per_c, auto reads_c) {
+        constexpr int PER = decltype(per_c)::value;
+        constexpr bool READS = decltype(reads_c)::value;
 #pragma unroll
-            for (int j = 0; j < FN; j++)
-                bf[j] = *reinterpret_cast<const i32x4*>(bb + j * 32 * LDSR + ks * 32);
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int j = 0; j < FN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
+        for (int q = 0; q < QS; q++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+            if constexpr (PER > 0) __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);  // VALU
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if constexpr (READS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+            if constexpr (PER > 0) __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);
         }
-        if ((s + 1) % SPG == 0) {
-            const int g = s / SPG;
-            float wsv[FN];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // FIRST: the step opens its group; LAST: it closes it (half 0 is folded here,
+    // half 1 beside the next group's first products)
+    auto step = [&](int s, auto first_c, auto last_c) {
+        constexpr bool FIRST = decltype(first_c)::value, LAST = decltype(last_c)::value;
+        const int8_t* ab = smem + (s & 1) * STAGE + (wm * 64) * LDSR + fo;
+        const int8_t* bb = smem + (s & 1) * STAGE + (BM + wn * 64) * LDSR + fo;
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < FN; j++) wsv[j] = wsc[j][g];
+        for (int u = 0; u < UPS; u++) {
+            i32x4 a0[QS], a1[QS], bf[2][QS];
 #pragma unroll
-            for (int i = 0; i < FM; i++)
+            for (int q = 0; q < QS; q++) {
+                a0[q] = *reinterpret_cast<const i32x4*>(ab + u * UK + q * 32);
 #pragma unroll
-                for (int j = 0; j < FN; j++) {
+                for (int j = 0; j < 2; j++)
+                    bf[j][q] = *reinterpret_cast<const i32x4*>(bb + j * 32 * LDSR + u * UK + q * 32);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            products(C0{}, first_c, a0, bf);
 #pragma unroll
-                    for (int r = 0; r < 16; r++)
-                        accf[i][j][r] = __builtin_fmaf((float)acc[i][j][r], wsv[j], accf[i][j][r]);
-                    acc[i][j] = i32x16{};
-                }
+            for (int q = 0; q < QS; q++)
+                a1[q] = *reinterpret_cast<const i32x4*>(ab + 32 * LDSR + u * UK + q * 32);
+            if constexpr (FIRST) fold(C1{}, wold);
+            interleave(std::integral_constant<int, FIRST ? 32 / QS : 0>{}, std::true_type{});
+            products(C1{}, first_c, a1, bf);
+            if constexpr (LAST) {
+                fold(C0{}, wnow[u]);
+                wold[0] = wnow[u][0];
+                wold[1] = wnow[u][1];
+            }
+            interleave(std::integral_constant<int, LAST ? 32 / QS : 0>{}, std::false_type{});
         }
-        __syncthreads();
-    }
+    };
 
+    gload(0);
+    wload(0);
+    wtake();
+    sstore(0);
+    lds_barrier();
+    // Every step but the last; straight-line code (a branch inside would let the
+    // compiler move the folds out of the products' shadow).
+    auto advance = [&](int s, auto first_c, auto last_c) {
+        constexpr bool LAST = decltype(last_c)::value;
+        gload(s + 1);
+        if constexpr (LAST) wload(s + 1);
+        step(s, first_c, last_c);
+        if constexpr (LAST) wtake();
+        sstore((s + 1) & 1);  // that stage was read in step s - 1, before the last barrier
+        lds_barrier();
+    };
+    if constexpr (SPG == 1) {
+        for (int s = 0; s < nsteps - 1; s++) advance(s, std::true_type{}, std::true_type{});
+        step(nsteps - 1, std::true_type{}, std::true_type{});
+    } else {
+        for (int s = 0; s < nsteps - 2; s += 2) {
+            advance(s, std::true_type{}, std::false_type{});
+            advance(s + 1, std::false_type{}, std::true_type{});
+        }
+        advance(nsteps - 2, std::true_type{}, std::false_type{});
+        step(nsteps - 1, std::false_type{}, std::true_type{});
+    }
+    fold(C1{}, wold);
+
+    // Epilogue: the tile's row scales go to LDS, the fp16 tile is staged there and
+    // leaves as 16-byte row chunks.
+    __syncthreads();  // every wave is done with the stages
+    float* scl = reinterpret_cast<float*>(smem + BM * kTileRow);
+    if (tid < BM) scl[tid] = m0 + tid < mend ? xs[src_row(m0 + tid)] : 0.0f;
+    float bcol[2] = {0.0f, 0.0f};
+    const bool has_bias = bias != nullptr;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int n = n0 + wn * 64 + j * 32 + (lane & 31);
+        if (has_bias && n < N) bcol[j] = fni8::h2f(bias[n]);
+    }
+    __syncthreads();
     // lane l, register r of block (i, j): row 8*(r/4) + 4*(l/32) + r%4, column l%32
 #pragma unroll
-    for (int i = 0; i < FM; i++)
+    for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int mr = m0 + wm * WTM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (mr >= mend) continue;
-            const float asc = xs[src_row(mr)];
+        for (int q = 0; q < 4; q++) {
+            const int row = wm * 64 + i * 32 + 8 * q + 4 * (lane >> 5);
+            const float4 a4 = *reinterpret_cast<const float4*>(scl + row);
+            const float asc[4] = {a4.x, a4.y, a4.z, a4.w};
 #pragma unroll
-            for (int j = 0; j < FN; j++) {
-                const int n = n0 + wn * WTN + j * 32 + (lane & 31);
-                if (n >= N) continue;
-                float v = accf[i][j][r] * asc;
-                if (bias) v = v + fni8::h2f(bias[n]);
-                y[(int64_t)mr * ldy + n] = fni8::f2h(v);
-            }
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    float v = accf[i][j][4 * q + r] * 0.0625f;
+                    v = v * asc[r];
+                    if (has_bias) v = v + bcol[j];
+                    const int col = wn * 64 + j * 32 + (lane & 31);
+                    *reinterpret_cast<uint16_t*>(smem + (row + r) * kTileRow + 2 * col) = fni8::f2h(v);
+                }
         }
+    __syncthreads();
+    const int col = n0 + (tid & 15) * 8;
+    if (col >= N) return;
+#pragma unroll
+    for (int it = 0; it < BM / 16; it++) {
+        const int row = it * 16 + (tid >> 4);
+        if (m0 + row >= mend) break;
+        const i32x4 v = *reinterpret_cast<const i32x4*>(smem + row * kTileRow + (tid & 15) * 16);
+        uint16_t* yp = y + (int64_t)(m0 + row) * ldy + col;
+        if (col + 7 < N && ((uintptr_t)yp & 15) == 0) {
+            *reinterpret_cast<i32x4*>(yp) = v;
+        } else {
+            for (int t = 0; t < 8 && col + t < N; t++)
+                yp[t] = (uint16_t)((uint32_t)v[t >> 1] >> (16 * (t & 1)));
+        }
+    }
 }
 
 // ---- prefill: 8-wave MFMA tile, two LDS stages -------------------------------
@@ -987,30 +1112,47 @@ int gemv_by_group(int64_t G, const int8_t* xq, int64_t ldq, const float* xs, int
     }
 }
 
-template <int G>
-int tile_launch(const int8_t* xq, int64_t ldq, const float* xs, int64_t M, int64_t K,
-                const uint8_t* w, const float* ws, int64_t N, const uint16_t* bias, uint16_t* y,
-                int64_t ldy, hipStream_t st) {
-    constexpr int BM = 128, BN = 128;
-    const dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((M + BM - 1) / BM));
-    hipLaunchKernelGGL((w4a8_tile_kernel<BM, BN, G>), grid, dim3(256), 0, st, xq, ldq, xs, nullptr,
-                       (int)M, (int)K, w, ws, (int)N, 0, nullptr, bias, y, ldy);
+// The kernel of a shape: steps of 128 codes (64 for groups of 32) where they divide
+// K, else of G codes.  Dense: 1-D grid, tiles in XCD order.  Grouped: activation rows of
+// stride K, y of stride N; the grid's x dimension bounds the segment tiles (sum
+// over experts of ceil(len / 128) <= M / 128 + E), its y dimension the column tiles.
+template <int G, int KS, bool GROUPED>
+int tile_launch_ks(const int8_t* xq, int64_t ldq, const float* xs, const int32_t* rmap, int64_t M,
+                   int64_t K, const uint8_t* w, const float* ws, int64_t N, int64_t E,
+                   const int32_t* seg_off, const uint16_t* bias, uint16_t* y, int64_t ldy,
+                   hipStream_t st) {
+    constexpr size_t lds = tile_lds<KS>();
+    const auto kern = &w4a8_tile_kernel<G, KS, GROUPED>;
+    if constexpr (lds > 64 * 1024) {
+        static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   (int)lds) == hipSuccess;
+        if (!ok) {
+            fni8h::set_error_detail("w4a8 tile: cannot raise the LDS limit to %zu bytes", lds);
+            return FNI8_ERR_LAUNCH;
+        }
+    }
+    const unsigned mt = (unsigned)((M + 127) / 128), nt = (unsigned)((N + 127) / 128);
+    const dim3 grid = GROUPED ? dim3(mt + (unsigned)E, nt) : dim3(mt * nt);
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, xq, ldq, xs, rmap, (int)M, (int)K, w, ws,
+                       (int)N, (int)E, seg_off, bias, y, ldy);
     return launch_error("w4a8 tile");
 }
 
-// Grouped form: activation rows of stride K, y of stride N; the grid's x
-// dimension bounds the segment tiles (sum over experts of ceil(len / 128) <=
-// R_max / 128 + E), its y dimension the column tiles.
-template <int G>
-int tile_grouped_launch(const int8_t* aq, const float* as, const int32_t* rmap, int64_t R_max,
-                        int64_t K, const uint8_t* w, const float* ws, int64_t E, int64_t N,
-                        const int32_t* seg_off, const uint16_t* bias, uint16_t* y,
-                        hipStream_t st) {
-    constexpr int BM = 128, BN = 128;
-    const dim3 grid((unsigned)((R_max + BM - 1) / BM + E), (unsigned)((N + BN - 1) / BN));
-    hipLaunchKernelGGL((w4a8_tile_kernel<BM, BN, G, true>), grid, dim3(256), 0, st, aq, K, as,
-                       rmap, (int)R_max, (int)K, w, ws, (int)N, (int)E, seg_off, bias, y, N);
-    return launch_error("w4a8 grouped tile");
+template <int G, bool GROUPED>
+int tile_launch(const int8_t* xq, int64_t ldq, const float* xs, const int32_t* rmap, int64_t M,
+                int64_t K, const uint8_t* w, const float* ws, int64_t N, int64_t E,
+                const int32_t* seg_off, const uint16_t* bias, uint16_t* y, int64_t ldy,
+                hipStream_t st) {
+    // a step of four groups of 32 does not fit the registers
+    constexpr int KS = G == 32 ? 64 : 128;
+    if constexpr (G < 128 && !GROUPED) {
+        if (K % KS != 0)
+            return tile_launch_ks<G, G, GROUPED>(xq, ldq, xs, rmap, M, K, w, ws, N, E, seg_off,
+                                                 bias, y, ldy, st);
+    }
+    return tile_launch_ks<G, KS, GROUPED>(xq, ldq, xs, rmap, M, K, w, ws, N, E, seg_off, bias, y,
+                                           ldy, st);
 }
 
 template <int G>
@@ -1276,9 +1418,9 @@ int launch_gemm_w4a8(const int8_t* xq, int64_t ldq, const float* xs, int64_t M, 
         }
     }
     switch (G) {
-        case 32: return tile_launch<32>(xq, ldq, xs, M, K, w, ws, N, bias, y, ldy, st);
-        case 64: return tile_launch<64>(xq, ldq, xs, M, K, w, ws, N, bias, y, ldy, st);
-        case 128: return tile_launch<128>(xq, ldq, xs, M, K, w, ws, N, bias, y, ldy, st);
+        case 32: return tile_launch<32, false>(xq, ldq, xs, nullptr, M, K, w, ws, N, 0, nullptr, bias, y, ldy, st);
+        case 64: return tile_launch<64, false>(xq, ldq, xs, nullptr, M, K, w, ws, N, 0, nullptr, bias, y, ldy, st);
+        case 128: return tile_launch<128, false>(xq, ldq, xs, nullptr, M, K, w, ws, N, 0, nullptr, bias, y, ldy, st);
         // G = 256 folds every other step: the 8-wave two-stage kernel is 6-35%
         // faster there (Qwen3-8B shapes at 2048 tokens).  At G <= 128 it folds
         // every step with all eight waves in lockstep, one workgroup per CU, and
@@ -1292,9 +1434,9 @@ int launch_w4a8_tile_grouped(const int8_t* aq, const float* as, const int32_t* r
                              int64_t E, int64_t N, int64_t G, const int32_t* seg_off,
                              const uint16_t* bias, uint16_t* y, hipStream_t st) {
     switch (G) {
-        case 64: return tile_grouped_launch<64>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, st);
-        case 128: return tile_grouped_launch<128>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, st);
-        default: return tile_grouped_launch<256>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, st);
+        case 64: return tile_launch<64, true>(aq, K, as, row_index, R_max, K, w, ws, N, E, seg_off, bias, y, N, st);
+        case 128: return tile_launch<128, true>(aq, K, as, row_index, R_max, K, w, ws, N, E, seg_off, bias, y, N, st);
+        default: return tile_launch<256, true>(aq, K, as, row_index, R_max, K, w, ws, N, E, seg_off, bias, y, N, st);
     }
 }
 
