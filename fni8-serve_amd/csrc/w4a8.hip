@@ -599,8 +599,9 @@ __global__ __launch_bounds__(WAVES * 64) void w4a8_mfma_kernel(
 //
 // Workgroup of 4 waves (2 x 2) over a 128 x 128 tile; each wave a 64 x 64 block,
 // as 2 x 2 blocks of 32x32.  K is consumed in steps of KS codes through two LDS
-// stages with one barrier a step: the next step's global loads are in flight
-// during the current step and go to the other stage at its end.  The packed
+// stages with one barrier a step: while a step's first fragments come from one
+// stage, the next step's operands go to the other, and the loads of the step after
+// that are issued.  The packed
 // weights are unpacked on the way to LDS, each nibble into the high half of its
 // byte (16 * code, natural k order), so the activations are stored unchanged.
 //
@@ -630,6 +631,12 @@ constexpr size_t tile_lds() {
     return stages > out ? stages : out;
 }
 
+// One 16-byte chunk per lane, global -> LDS at lds + lane * 16 (wave-uniform lds).
+__device__ __forceinline__ void copy16_lds(uint32_t lds, const int8_t* src) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :: "s"(lds), "v"(src) : "memory", "m0");
+}
+
 template <int G, int KS, bool GROUPED = false>
 __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
     const int8_t* __restrict__ xq, int64_t ldq, const float* __restrict__ xs,
@@ -642,7 +649,11 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
     constexpr int SPG = G / UK;             // steps per group
     constexpr int QS = UK / 32;             // MFMAs per block and unit
     constexpr int LDSR = KS + 16;           // padded LDS row (bytes)
-    constexpr int STAGE = (BM + BN) * LDSR;
+    // 128-code steps: the activations go straight to LDS (global_load_lds), their
+    // 128-byte rows unpadded with the 16-byte chunks of row r at c ^ ((r / 2) % 8)
+    constexpr bool DIRECT = KS == 128;
+    constexpr int ROWA = DIRECT ? KS : LDSR;
+    constexpr int STAGE = BM * ROWA + BN * LDSR;
     constexpr int A_TOT = BM * (KS / 16), B_TOT = BN * (KS / 32);  // 16-byte chunks per step
     constexpr int A_CH = (A_TOT + NT - 1) / NT, B_CH = (B_TOT + NT - 1) / NT;
     static_assert(SPG == 1 || (UPS == 1 && SPG == 2), "a step holds whole groups or half of one");
@@ -677,10 +688,14 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
     const uint8_t* bsrc[B_CH];
 #pragma unroll
     for (int i = 0; i < A_CH; i++) {
-        const int c = (tid + i * NT) % A_TOT;  // threads past the step's chunks repeat one
-        int mr = m0 + c / (KS / 16);
+        // direct: copy i of this wave fills rows (wave * A_CH + i) * 8 .. + 8
+        const int c = DIRECT ? (wave * A_CH + i) * 64 + lane
+                             : (tid + i * NT) % A_TOT;  // threads past the step's chunks repeat one
+        const int row = c / (KS / 16);
+        int mr = m0 + row;
         mr = mr < mend ? mr : mend - 1;
-        asrc[i] = xq + (int64_t)src_row(mr) * ldq + (c % (KS / 16)) * 16;
+        const int chunk = DIRECT ? (c % 8) ^ ((row >> 1) & 7) : c % (KS / 16);
+        asrc[i] = xq + (int64_t)src_row(mr) * ldq + chunk * 16;
     }
 #pragma unroll
     for (int i = 0; i < B_CH; i++) {
@@ -690,26 +705,42 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
         bsrc[i] = w + (int64_t)nr * (K / 2) + (c % (KS / 32)) * 16;
     }
     i32x4 ra[A_CH], rb[B_CH];
-    auto gload = [&](int s) {
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+    auto acopy = [&](int s, int buf) {  // completion: wait_copies
+        if constexpr (DIRECT) {
 #pragma unroll
-        for (int i = 0; i < A_CH; i++) ra[i] = *reinterpret_cast<const i32x4*>(asrc[i] + (int64_t)s * KS);
+            for (int i = 0; i < A_CH; i++)
+                copy16_lds(lds0 + buf * STAGE + (wave * A_CH + i) * 1024, asrc[i] + (int64_t)s * KS);
+        }
+    };
+    auto wait_copies = [&]() {
+        if constexpr (DIRECT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    auto gload = [&](int s) {
+        if constexpr (!DIRECT) {
+#pragma unroll
+            for (int i = 0; i < A_CH; i++)
+                ra[i] = *reinterpret_cast<const i32x4*>(asrc[i] + (int64_t)s * KS);
+        }
 #pragma unroll
         for (int i = 0; i < B_CH; i++)
             rb[i] = *reinterpret_cast<const i32x4*>(bsrc[i] + (int64_t)s * (KS / 2));
     };
     auto sstore = [&](int buf) {
         int8_t* st = smem + buf * STAGE;
+        if constexpr (!DIRECT) {
 #pragma unroll
-        for (int i = 0; i < A_CH; i++) {
-            const int c = tid + i * NT;
-            if (A_TOT % NT != 0 && c >= A_TOT) continue;
-            *reinterpret_cast<i32x4*>(st + (c / (KS / 16)) * LDSR + (c % (KS / 16)) * 16) = ra[i];
+            for (int i = 0; i < A_CH; i++) {
+                const int c = tid + i * NT;
+                if (A_TOT % NT != 0 && c >= A_TOT) continue;
+                *reinterpret_cast<i32x4*>(st + (c / (KS / 16)) * ROWA + (c % (KS / 16)) * 16) = ra[i];
+            }
         }
 #pragma unroll
         for (int i = 0; i < B_CH; i++) {
             const int c = tid + i * NT;
             if (B_TOT % NT != 0 && c >= B_TOT) continue;
-            int8_t* dst = st + (BM + c / (KS / 32)) * LDSR + (c % (KS / 32)) * 32;
+            int8_t* dst = st + BM * ROWA + (c / (KS / 32)) * LDSR + (c % (KS / 32)) * 32;
             *reinterpret_cast<i32x4*>(dst) = unpack16x16(rb[i][0], rb[i][1]);
             *reinterpret_cast<i32x4*>(dst + 16) = unpack16x16(rb[i][2], rb[i][3]);
         }
@@ -759,6 +790,11 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
     // fragment read: lane l takes row l % 32 of a 32-row block and bytes
     // 16 * (l / 32) of each 32-byte sub-step (the 32x32x32 operand layout)
     const int fo = (lane & 31) * LDSR + (lane >> 5) * 16;
+    int fa[KS / 32];  // of an activation block, by sub-step
+#pragma unroll
+    for (int q = 0; q < KS / 32; q++)
+        fa[q] = DIRECT ? (lane & 31) * ROWA + (((2 * q + (lane >> 5)) ^ ((lane >> 1) & 7)) & 7) * 16
+                       : fo + q * 32;
     auto products = [&](auto half_c, auto first_c, const i32x4 (&af)[QS], const i32x4 (&bf)[2][QS]) {
         constexpr int i = decltype(half_c)::value;
 #pragma unroll
@@ -788,26 +824,30 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
     };
     // FIRST: the step opens its group; LAST: it closes it (half 0 is folded here,
     // half 1 beside the next group's first products)
-    auto step = [&](int s, auto first_c, auto last_c) {
+    auto step = [&](int s, auto first_c, auto last_c, auto staging) {
         constexpr bool FIRST = decltype(first_c)::value, LAST = decltype(last_c)::value;
-        const int8_t* ab = smem + (s & 1) * STAGE + (wm * 64) * LDSR + fo;
-        const int8_t* bb = smem + (s & 1) * STAGE + (BM + wn * 64) * LDSR + fo;
+        const int8_t* ab = smem + (s & 1) * STAGE + (wm * 64) * ROWA;
+        const int8_t* bb = smem + (s & 1) * STAGE + BM * ROWA + (wn * 64) * LDSR + fo;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < UPS; u++) {
             i32x4 a0[QS], a1[QS], bf[2][QS];
 #pragma unroll
             for (int q = 0; q < QS; q++) {
-                a0[q] = *reinterpret_cast<const i32x4*>(ab + u * UK + q * 32);
+                a0[q] = *reinterpret_cast<const i32x4*>(ab + fa[u * QS + q]);
 #pragma unroll
                 for (int j = 0; j < 2; j++)
                     bf[j][q] = *reinterpret_cast<const i32x4*>(bb + j * 32 * LDSR + u * UK + q * 32);
             }
             __builtin_amdgcn_sched_barrier(0);
+            if (u == 0) {
+                staging();  // while the fragments come
+                __builtin_amdgcn_sched_barrier(0);
+            }
             products(C0{}, first_c, a0, bf);
 #pragma unroll
             for (int q = 0; q < QS; q++)
-                a1[q] = *reinterpret_cast<const i32x4*>(ab + 32 * LDSR + u * UK + q * 32);
+                a1[q] = *reinterpret_cast<const i32x4*>(ab + 32 * ROWA + fa[u * QS + q]);
             if constexpr (FIRST) fold(C1{}, wold);
             interleave(std::integral_constant<int, FIRST ? 32 / QS : 0>{}, std::true_type{});
             products(C1{}, first_c, a1, bf);
@@ -820,32 +860,44 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
         }
     };
 
+    // Step s stores the operands of step s + 1 (loaded a step ago) into the stage
+    // that step s - 1 read, before the last barrier, and loads those of step s + 2
+    // (the last ones again past the end).
     gload(0);
     wload(0);
     wtake();
     sstore(0);
+    acopy(0, 0);
+    gload(nsteps > 1 ? 1 : 0);
+    wait_copies();
     lds_barrier();
     // Every step but the last; straight-line code (a branch inside would let the
     // compiler move the folds out of the products' shadow).
     auto advance = [&](int s, auto first_c, auto last_c) {
         constexpr bool LAST = decltype(last_c)::value;
-        gload(s + 1);
-        if constexpr (LAST) wload(s + 1);
-        step(s, first_c, last_c);
+        step(s, first_c, last_c, [&]() {
+            // the weights first: the compiler's wait for them must not see the copies
+            sstore((s + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
+            acopy(s + 1, (s + 1) & 1);
+            gload(s + 2 < nsteps ? s + 2 : nsteps - 1);
+            if constexpr (LAST) wload(s + 1);
+        });
         if constexpr (LAST) wtake();
-        sstore((s + 1) & 1);  // that stage was read in step s - 1, before the last barrier
+        wait_copies();
         lds_barrier();
     };
+    const auto idle = [] {};
     if constexpr (SPG == 1) {
         for (int s = 0; s < nsteps - 1; s++) advance(s, std::true_type{}, std::true_type{});
-        step(nsteps - 1, std::true_type{}, std::true_type{});
+        step(nsteps - 1, std::true_type{}, std::true_type{}, idle);
     } else {
         for (int s = 0; s < nsteps - 2; s += 2) {
             advance(s, std::true_type{}, std::false_type{});
             advance(s + 1, std::false_type{}, std::true_type{});
         }
         advance(nsteps - 2, std::true_type{}, std::false_type{});
-        step(nsteps - 1, std::false_type{}, std::true_type{});
+        step(nsteps - 1, std::false_type{}, std::true_type{}, idle);
     }
     fold(C1{}, wold);
 
@@ -897,168 +949,6 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
                 yp[t] = (uint16_t)((uint32_t)v[t >> 1] >> (16 * (t & 1)));
         }
     }
-}
-
-// ---- prefill: 8-wave MFMA tile, two LDS stages -------------------------------
-//
-// The W8A8 prefill pipeline (8 waves as 2 x 4, two LDS stages, global loads
-// staged in registers, LDS-only barriers) with the group-wise fold.  A BM x BN
-// = 128 x 256 tile gives each wave a 64 x 64 block: int32 accumulators for the
-// current group plus fp32 running sums, 128 registers.  A K-step is KS =
-// min(G, 128) codes.  The packed weight step is unpacked as it goes to LDS,
-// each nibble into the high half of its byte (16 * code, natural k order), so
-// the activations go to LDS unchanged; the sums come out 16x and an
-// arithmetic shift restores them exactly before the fold.  With two waves per
-// SIMD, one wave's fold overlaps the other's MFMAs.
-template <int BM, int BN, int G>
-__global__ __launch_bounds__(512) void w4a8_tile8_kernel(
-    const int8_t* __restrict__ xq, int64_t ldq, const float* __restrict__ xs, int M, int K,
-    const uint8_t* __restrict__ w, const float* __restrict__ ws, int N,
-    const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t ldy) {
-    constexpr int NT = 512;
-    constexpr int KS = G < 128 ? G : 128;  // codes per K-step
-    constexpr int SPG = G / KS;            // steps per group
-    constexpr int LDSR = KS + 16;          // padded LDS row (bytes)
-    constexpr int WTM = BM / 2, WTN = BN / 4;
-    constexpr int FM = WTM / 32, FN = WTN / 32;
-    constexpr int A_TOT = BM * (KS / 16), B_TOT = BN * (KS / 32);  // 16-byte chunks per step
-    constexpr int A_CH = (A_TOT + NT - 1) / NT, B_CH = (B_TOT + NT - 1) / NT;
-    constexpr int STAGE = (BM + BN) * LDSR;
-    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 2, wn = wave & 3;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int ng = K / G, nsteps = K / KS;
-
-    // rows past the end repeat the last valid row (their results are never
-    // stored); threads past a step's chunk count repeat a chunk and skip the store
-    const int8_t* asrc[A_CH];
-    const uint8_t* bsrc[B_CH];
-#pragma unroll
-    for (int i = 0; i < A_CH; i++) {
-        const int c = (tid + i * NT) % A_TOT;
-        int mr = m0 + c / (KS / 16);
-        mr = mr < M ? mr : M - 1;
-        asrc[i] = xq + (int64_t)mr * ldq + (c % (KS / 16)) * 16;
-    }
-#pragma unroll
-    for (int i = 0; i < B_CH; i++) {
-        const int c = (tid + i * NT) % B_TOT;
-        int nr = n0 + c / (KS / 32);
-        nr = nr < N ? nr : N - 1;
-        bsrc[i] = w + (int64_t)nr * (K / 2) + (c % (KS / 32)) * 16;
-    }
-    uint4 ra[A_CH], rb[B_CH];
-    auto gload = [&](int s) {
-#pragma unroll
-        for (int i = 0; i < A_CH; i++) ra[i] = *reinterpret_cast<const uint4*>(asrc[i] + (int64_t)s * KS);
-#pragma unroll
-        for (int i = 0; i < B_CH; i++)
-            rb[i] = *reinterpret_cast<const uint4*>(bsrc[i] + (int64_t)s * (KS / 2));
-    };
-    auto sstore = [&](int buf) {
-        int8_t* st = smem + buf * STAGE;
-#pragma unroll
-        for (int i = 0; i < A_CH; i++) {
-            const int c = tid + i * NT;
-            if (A_TOT % NT != 0 && c >= A_TOT) continue;
-            *reinterpret_cast<uint4*>(st + (c / (KS / 16)) * LDSR + (c % (KS / 16)) * 16) = ra[i];
-        }
-#pragma unroll
-        for (int i = 0; i < B_CH; i++) {
-            const int c = tid + i * NT;
-            if (B_TOT % NT != 0 && c >= B_TOT) continue;
-            int8_t* dst = st + (BM + c / (KS / 32)) * LDSR + (c % (KS / 32)) * 32;
-            *reinterpret_cast<i32x4*>(dst) = unpack16x16(rb[i].x, rb[i].y);
-            *reinterpret_cast<i32x4*>(dst + 16) = unpack16x16(rb[i].z, rb[i].w);
-        }
-    };
-
-    i32x16 acc[FM][FN];
-    float accf[FM][FN][16];
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-            acc[i][j] = i32x16{};
-#pragma unroll
-            for (int r = 0; r < 16; r++) accf[i][j][r] = 0.0f;
-        }
-    const float* wsc[FN];
-#pragma unroll
-    for (int j = 0; j < FN; j++) {
-        int n = n0 + wn * WTN + j * 32 + (lane & 31);
-        n = n < N ? n : N - 1;
-        wsc[j] = ws + (int64_t)n * ng;
-    }
-
-    // fragment read: lane l takes row l % 32 of a 32-row block and bytes
-    // 16 * (l / 32) of each 32-byte sub-step (the 32x32x32 operand layout)
-    const int fo = (lane & 31) * LDSR + (lane >> 5) * 16;
-    auto compute = [&](int buf) {
-        const int8_t* ab = smem + buf * STAGE + (wm * WTM) * LDSR + fo;
-        const int8_t* bb = smem + buf * STAGE + (BM + wn * WTN) * LDSR + fo;
-#pragma unroll
-        for (int ks = 0; ks < KS / 32; ks++) {
-            i32x4 af[FM], bf[FN];
-#pragma unroll
-            for (int i = 0; i < FM; i++) af[i] = *reinterpret_cast<const i32x4*>(ab + i * 32 * LDSR + ks * 32);
-#pragma unroll
-            for (int j = 0; j < FN; j++) bf[j] = *reinterpret_cast<const i32x4*>(bb + j * 32 * LDSR + ks * 32);
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int j = 0; j < FN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-    };
-    auto fold = [&](int g) {
-        float wsv[FN];
-#pragma unroll
-        for (int j = 0; j < FN; j++) wsv[j] = wsc[j][g];
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-            for (int j = 0; j < FN; j++) {
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    accf[i][j][r] = __builtin_fmaf((float)(acc[i][j][r] >> 4), wsv[j], accf[i][j][r]);
-                acc[i][j] = i32x16{};
-            }
-    };
-
-    gload(0);
-    sstore(0);
-    if (nsteps > 1) gload(1);
-    lds_barrier();
-    for (int s = 0; s < nsteps; s++) {
-        compute(s & 1);
-        if ((s + 1) % SPG == 0) fold(s / SPG);
-        if (s + 1 < nsteps) {
-            sstore((s + 1) & 1);  // that stage was read by step s - 1, before the last barrier
-            if (s + 2 < nsteps) gload(s + 2);
-        }
-        lds_barrier();
-    }
-
-    // lane l, register r of block (i, j): row 8*(r/4) + 4*(l/32) + r%4, column l%32
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int mr = m0 + wm * WTM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (mr >= M) continue;
-            const float asc = xs[mr];
-#pragma unroll
-            for (int j = 0; j < FN; j++) {
-                const int n = n0 + wn * WTN + j * 32 + (lane & 31);
-                if (n >= N) continue;
-                float v = accf[i][j][r] * asc;
-                if (bias) v = v + fni8::h2f(bias[n]);
-                y[(int64_t)mr * ldy + n] = fni8::f2h(v);
-            }
-        }
 }
 
 int launch_error(const char* what) {
@@ -1153,26 +1043,6 @@ int tile_launch(const int8_t* xq, int64_t ldq, const float* xs, const int32_t* r
     }
     return tile_launch_ks<G, KS, GROUPED>(xq, ldq, xs, rmap, M, K, w, ws, N, E, seg_off, bias, y,
                                            ldy, st);
-}
-
-template <int G>
-int tile8_launch(const int8_t* xq, int64_t ldq, const float* xs, int64_t M, int64_t K,
-                 const uint8_t* w, const float* ws, int64_t N, const uint16_t* bias, uint16_t* y,
-                 int64_t ldy, hipStream_t st) {
-    constexpr int BM = 128, BN = 256, KS = G < 128 ? G : 128;
-    constexpr size_t lds = (size_t)2 * (BM + BN) * (KS + 16);
-    auto kern = &w4a8_tile8_kernel<BM, BN, G>;
-    static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)lds) == hipSuccess;
-    if (!ok) {
-        fni8h::set_error_detail("w4a8 tile: cannot raise the LDS limit to %zu bytes", lds);
-        return FNI8_ERR_LAUNCH;
-    }
-    const dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((M + BM - 1) / BM));
-    hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, xq, ldq, xs, (int)M, (int)K, w, ws, (int)N,
-                       bias, y, ldy);
-    return launch_error("w4a8 tile");
 }
 
 // LDS bytes of w4a8_stream_kernel: activations, group sums, scales.
@@ -1421,11 +1291,7 @@ int launch_gemm_w4a8(const int8_t* xq, int64_t ldq, const float* xs, int64_t M, 
         case 32: return tile_launch<32, false>(xq, ldq, xs, nullptr, M, K, w, ws, N, 0, nullptr, bias, y, ldy, st);
         case 64: return tile_launch<64, false>(xq, ldq, xs, nullptr, M, K, w, ws, N, 0, nullptr, bias, y, ldy, st);
         case 128: return tile_launch<128, false>(xq, ldq, xs, nullptr, M, K, w, ws, N, 0, nullptr, bias, y, ldy, st);
-        // G = 256 folds every other step: the 8-wave two-stage kernel is 6-35%
-        // faster there (Qwen3-8B shapes at 2048 tokens).  At G <= 128 it folds
-        // every step with all eight waves in lockstep, one workgroup per CU, and
-        // is 30-45% slower than the 4-wave kernel, which fits two workgroups.
-        default: return tile8_launch<256>(xq, ldq, xs, M, K, w, ws, N, bias, y, ldy, st);
+        default: return tile_launch<256, false>(xq, ldq, xs, nullptr, M, K, w, ws, N, 0, nullptr, bias, y, ldy, st);
     }
 }
 
