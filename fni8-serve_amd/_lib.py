@@ -50,6 +50,7 @@ INT64_FUNCS = {"fni8_linear_workspace_bytes": [_I, _I, _I],
 VOID_FUNCS = {"fni8_debug_coop_wait_ticks": [_I], "fni8_debug_gemm_plan": [_I, _I, _I]}
 
 _lib = None
+_host = None
 _lock = threading.Lock()
 
 
@@ -86,6 +87,21 @@ def load() -> ctypes.CDLL:
             fn.restype = ctypes.c_int64
         _lib = lib
         return lib
+
+
+def host():
+    """The native host path (csrc/host.cpp, built next to the library); RuntimeError if
+    it is not there."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError(f"{os.path.join(_PKG_DIR, '_host.so')} does not load: build it with "
+                               f"`make -C {os.path.join(_PKG_DIR, 'csrc')}`") from e
+        _host = module
+    return _host
 
 
 def call(name: str, *args) -> None:

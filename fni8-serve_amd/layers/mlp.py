@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from .. import ops
 from ..qtensor import QTensor
@@ -28,6 +29,15 @@ from .linear import LinearW8A8
 FUSE_MIN_ROWS = 5
 
 
+def bare(m: nn.Module, cls: type) -> bool:
+    """True when calling `m` is calling cls.forward and nothing else: exactly that class,
+    no hook on it or on every module, no forward of its own."""
+    d = m.__dict__
+    return (type(m) is cls and "forward" not in d
+            and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                     or d["_backward_pre_hooks"] or _has_any_global_hook()))
+
+
 class GatedMLP(nn.Module):
     def __init__(self, gate_up: QTensor, down: QTensor, *, act: nn.Module | str = "silu",
                  bias_gate_up=None, bias_down=None):
@@ -40,6 +50,12 @@ class GatedMLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         act = fused_act(self.act_fn)
+        if (act is not None and x.is_cuda and bare(self.gate_up_proj, LinearW8A8)
+                and bare(self.down_proj, LinearW8A8) and bare(self.act_fn, type(self.act_fn))):
+            y = ops.gated_mlp(x, self.gate_up_proj.weight, self.down_proj.weight, act,
+                              self.gate_up_proj.bias, self.down_proj.bias, FUSE_MIN_ROWS)
+            if y is not None:
+                return y
         rows = x.numel() // max(x.shape[-1], 1)
         if (act is not None and rows >= FUSE_MIN_ROWS and self.gate_up_proj._int8_ok(x)
                 and self.down_proj._int8_ok(x)):

@@ -66,6 +66,10 @@ def _w4_stackable(qs: list[QTensor]) -> bool:
                for q in qs)
 
 
+# the steps that `_native` does in one call, unless an instance has its own
+_STEPS = ("route", "experts_grouped", "experts_grouped_w4")
+
+
 class SparseMoE(nn.Module):
     def __init__(self, *, gate: torch.Tensor, experts: list[tuple[QTensor, QTensor]], top_k: int,
                  norm_topk_prob: bool = True, act: str = "silu",
@@ -245,19 +249,33 @@ class SparseMoE(nn.Module):
             out.index_add_(0, tok_idx, contrib * topw[tok_idx, slot].unsqueeze(-1))
         return out
 
+    def _native(self, xf: torch.Tensor):
+        """route, experts_grouped and experts_grouped_w4 as one host call; None where
+        they have to run one by one."""
+        act = fused_act(self.act_fn)
+        if (act is None or type(self) is not SparseMoE or not (self.grouped or self.grouped_w4)
+                or not self.__dict__.keys().isdisjoint(_STEPS)):
+            return None
+        g1, g2 = (0, 0) if self.grouped else (self.g_gate_up, self.g_down)
+        return ops.sparse_moe(xf, self._gate_f32(), self.top_k, self.scoring_func,
+                              self.e_score_bias, self.num_expert_groups, self.topk_group,
+                              self.norm_topk_prob, self.routed_scaling_factor, self.w_gate_up,
+                              self.s_gate_up, g1, self.w_down, self.s_down, g2, act)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         B, S, H = x.shape
         xf = x.reshape(-1, H)
-        topw, topi = self.route(xf)
-        if xf.is_cuda:
-            if self.grouped:
+        out = self._native(xf) if xf.is_cuda else None
+        if out is None:
+            topw, topi = self.route(xf)
+            if not xf.is_cuda:
+                out = self._experts_loop(xf, topw, topi)
+            elif self.grouped:
                 out = self.experts_grouped(xf, topw, topi)
             elif self.grouped_w4:
                 out = self.experts_grouped_w4(xf, topw, topi)
             else:
                 out = self.experts_sorted(xf, topw, topi)
-        else:
-            out = self._experts_loop(xf, topw, topi)
         if self.shared is not None:
             shared_out = self.shared(x).reshape(-1, H)
             if self.shared_gate is not None:

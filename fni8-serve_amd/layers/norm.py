@@ -38,7 +38,7 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor, residual: torch.Tensor | None = None):
         if x.is_cuda and x.dtype == torch.float16 and self.weight.dtype == torch.float16:
-            return ops.rmsnorm(x, self.weight.detach(), self.eps, residual=residual,
+            return ops.rmsnorm(x, self.weight, self.eps, residual=residual,
                                unit_offset=self.add_unit_offset)
         if residual is None:
             return self._norm(x)
@@ -48,5 +48,5 @@ class RMSNorm(nn.Module):
     def forward_quant(self, x: torch.Tensor, residual: torch.Tensor | None = None):
         """(xq int8 [M, K], xs fp32 [M]) -- plus x + residual with a residual --
         bit-identical to quantizing forward(x, residual)'s normed output."""
-        return ops.rmsnorm_quant(x, self.weight.detach(), self.eps, residual=residual,
+        return ops.rmsnorm_quant(x, self.weight, self.eps, residual=residual,
                                  unit_offset=self.add_unit_offset)
