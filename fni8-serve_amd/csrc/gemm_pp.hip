@@ -459,6 +459,32 @@ bool pp_plan(int64_t M, int64_t N, int64_t K, int64_t work_bytes, PpPlan& out) {
         out = PpPlan{64, 128, 4, need};
         return true;
     }
+    // The same tile, three workgroups per CU, where the bigger ones leave the chip
+    // idle (us against the plan or kernel chosen below, weights from HBM):
+    //   M <= 128, K >= 3072: the deepest split that fits one round of 3 per CU
+    //     (M = 100: N x K = 4096 x 4096 12.5 : 15.9, 24576 x 4096 split 2 28.3 : 39.0,
+    //     1536 x 4608 11.3 : 16.2; at K <= 1536 every split was slower)
+    //   M <= 512: split 4 on one workgroup per CU (M = 500: 1024 x 3072 10.7 : 11.6), from
+    //     K = 4096 on two (M = 333: 1536 x 4608 13.3 : 16.0; 1536 x 3072, 384 workgroups,
+    //     12.5 : 11.9), for long K three (4096 x 12288 36.8 : 41.9; 4096 x 4096 18.2 : 17.2)
+    //   unsplit, K <= 4096: where it fills more than two and at most three per CU
+    //     (M = 777: 6144 x 4096 32.7 : 39.2, with 416 workgroups 27.1 : 22.9; longer K has
+    //     better split plans: M = 1536, 4096 x 12288 107 : 86)
+    const int64_t t64 = ((M + 63) / 64) * ((N + 127) / 128), kt64 = K / 128;
+    if (K >= 3072 && M <= 512) {
+        const int per_cu = M <= 128 || K >= 8192 ? 3 : K >= 4096 ? 2 : 1;
+        for (int split = 4; split >= (M <= 128 ? 2 : 4); split /= 2) {
+            if (kt64 / split >= 6 && t64 * split <= (int64_t)per_cu * cus &&
+                plan_valid(M, N, K, 64, 128, split, work_bytes, need)) {
+                out = PpPlan{64, 128, split, need};
+                return true;
+            }
+        }
+    }
+    if (K >= 1024 && K <= 4096 && t64 > 2 * cus && t64 <= 3 * cus) {
+        out = PpPlan{64, 128, 1, 0};
+        return true;
+    }
     // candidates in order of preference on equal estimates; of the half-size
     // tiles 256x128 first for long K and for a single row of tiles (M <= 256,
     // where it reads each weight row once: gate_up at M = 256 45 against 50 us)
