@@ -282,13 +282,13 @@ template <int G>
 int grouped_by_tile(const int8_t* aq, const float* as, const int32_t* rmap, int64_t R_max,
                     int64_t K, const uint8_t* w, const float* ws, int64_t E, int64_t N,
                     const int32_t* seg_off, const uint16_t* bias, uint16_t* y, hipStream_t st) {
-    // Segment tiles of 16, 32 or 64 rows by the mean rows per expert, four
+    // Segment tiles of 16 or 32 rows by the mean rows per expert, four
     // waves.  Measured on the Qwen3-30B-A3B projections (128 experts, top-8,
     // uniform routing; gate_up [1536, 2048], down [2048, 768]), µs against the
     // earlier 16-row, two-wave, two-slab shape: T = 16 gate_up 30.44 / 32.69,
     // down 18.87 / 21.97 (16-row tiles); T = 256 gate_up 62.61 / 81.28, down
     // 40.41 / 49.11 (32-row tiles).  One slab per batch was faster than two at
-    // every small-segment point; 64-row tiles keep two where K allows.
+    // every small-segment point.
     // With few rows (T = 1: 8 of 128 experts) four-wave workgroups would leave
     // the grid under two per CU; the two-wave shape stays there.
     const double avg = (double)R_max / (double)E;
@@ -302,13 +302,8 @@ int grouped_by_tile(const int8_t* aq, const float* as, const int32_t* rmap, int6
     if (avg <= 8.0)
         return rowblock_grouped_launch<1, 4, 1, G>(aq, as, rmap, R_max, K, w, ws, E, N, seg_off,
                                                    bias, y, st);
-    if (avg <= 32.0)
-        return rowblock_grouped_launch<2, 4, 1, G>(aq, as, rmap, R_max, K, w, ws, E, N, seg_off,
-                                                   bias, y, st);
-    return sb2 ? rowblock_grouped_launch<4, 4, 2, G>(aq, as, rmap, R_max, K, w, ws, E, N,
-                                                     seg_off, bias, y, st)
-               : rowblock_grouped_launch<4, 4, 1, G>(aq, as, rmap, R_max, K, w, ws, E, N,
-                                                     seg_off, bias, y, st);
+    return rowblock_grouped_launch<2, 4, 1, G>(aq, as, rmap, R_max, K, w, ws, E, N, seg_off, bias,
+                                               y, st);
 }
 
 }  // namespace
@@ -358,9 +353,12 @@ int launch_gemm_w4a8_grouped(const int8_t* aq, const float* as, const int32_t* r
                              int64_t E, int64_t N, int64_t G, const int32_t* seg_off,
                              const uint16_t* bias, uint16_t* y, hipStream_t st) {
     if (R_max == 0) return FNI8_OK;
-    // 64 or more rows per expert on average: 128x128 segment tiles of the
-    // prefill tile kernel (w4a8.hip)
-    if (R_max >= 64 * E)
+    // More than 32 rows per expert on average: 128x128 segment tiles of the prefill
+    // tile kernel (w4a8.hip).  gate_up + down of 128 experts, hidden 2048, inter 768,
+    // G = 128, us here : there, uniform routing / Zipf-skewed: 24 rows 128 : 147 /
+    // 147 : 137, 32 rows 155 : 148 / 168 : 148, 40 rows 182 : 151 / 226 : 169,
+    // 63 rows 267 : 159 / 290 : 195 (here: 64-row tiles above 32 rows).
+    if (R_max > 32 * E)
         return launch_w4a8_tile_grouped(aq, as, row_index, R_max, K, w, ws, E, N, G, seg_off,
                                         bias, y, st);
     switch (G) {
