@@ -367,7 +367,7 @@ __global__ __launch_bounds__(WAVES * 64) void w4a8_stream_kernel(
     }
 }
 
-// ---- decode on MFMA: int8 activations, up to 64 tokens -----------------------
+// ---- decode on MFMA: int8 activations, up to 64 tokens a slice -----------------
 //
 // The W8A8 decode layout with packed weights.  A workgroup owns 16*NB weight
 // rows.  One load instruction covers 8 rows x 128 packed bytes (a "slab" of
@@ -410,6 +410,13 @@ __global__ __launch_bounds__(WAVES * 64) void w4a8_mfma_kernel(
                       EL % (WAVES * 64) == 0, "w4a8 mfma shape");
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     int32_t* gs = reinterpret_cast<int32_t*>(smem + WAVES * SB * TILE);  // [2][GPR][EL]
+
+    // token slice blockIdx.y of TOK rows
+    const int m0 = blockIdx.y * TOK;
+    xq += (int64_t)m0 * ldx;
+    xs += m0;
+    y += (int64_t)m0 * ldy;
+    M = M - m0 < TOK ? M - m0 : TOK;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1096,7 +1103,8 @@ int mfma_launch(const int8_t* xq, int64_t ldq, const float* xs, int64_t M, int64
             return FNI8_ERR_LAUNCH;
         }
     }
-    const dim3 grid((unsigned)((N + 16 * NB - 1) / (16 * NB)));
+    const dim3 grid((unsigned)((N + 16 * NB - 1) / (16 * NB)),
+                    (unsigned)((M + 16 * MT - 1) / (16 * MT)));
     hipLaunchKernelGGL(kern, grid, dim3(WAVES * 64), lds, st, xq, ldq, xs, (int)M, (int)K, w, ws,
                        (int)N, bias, y, ldy);
     return launch_error("w4a8 mfma");
@@ -1131,14 +1139,29 @@ int mfma_table(const int8_t* xq, int64_t ldq, const float* xs, int64_t M, int64_
     return 1;
 }
 
-// 1 when the shape is not taken: group size 64..256, K a multiple of 256, at
-// most 64 tokens, 16-byte aligned activation rows.
+// 1 when the shape is not taken: group size 64..256, K a multiple of 256, 16-byte
+// aligned activation rows, and at most 64 tokens -- or more, in equal slices of at
+// most 64 side by side, while those are at most two workgroups of 16 weight rows per
+// CU (one for groups of 64, whose sums are twice as many).  The tile kernel's few
+// workgroups walk the whole K there (us, sliced : tile kernel, G = 128): 4096 x 4096
+// 65 tokens 18.9 : 32.3, 128 tokens 24.6 : 33.5; 4096 x 12288 100 tokens 60.5 : 118;
+// 1024 x 3072 256 tokens 9.9 : 24.7; 1536 x 4608 200 tokens 21.1 : 35.3.
 int mfma_dispatch(const int8_t* xq, int64_t ldq, const float* xs, int64_t M, int64_t K,
                   const uint8_t* w, const float* ws, int64_t N, int64_t G, const uint16_t* bias,
                   uint16_t* y, int64_t ldy, hipStream_t st) {
-    if (M < 1 || M > 64 || G < 64 || K % 256 != 0 || K > 65536) return 1;
+    if (M < 1 || G < 64 || K % 256 != 0 || K > 65536) return 1;
     if (ldq % 16 != 0 || ((uintptr_t)xq % 16) != 0 || ((uintptr_t)w % 16) != 0) return 1;
-    const int mt = (int)((M + 15) / 16);
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            n <= 0)
+            n = 256;
+        return n;
+    }();
+    const int64_t slices = (M + 63) / 64;
+    if (slices > 1 && (N + 15) / 16 * slices > (G == 64 ? 1 : 2) * (int64_t)cus) return 1;
+    const int mt = (int)((M + 16 * slices - 1) / (16 * slices));
 #define FNI8_W4M_G(MTV)                                                                         \
     switch (G) {                                                                                \
         case 64: return mfma_table<MTV, 64>(xq, ldq, xs, M, K, w, ws, N, bias, y, ldy, st);     \
