@@ -6,11 +6,13 @@
 // allocate the outputs and one scratch buffer per call, and make the C ABI calls of
 // a whole chain (linear, norm, MLP, MoE) from one Python call.
 //
-// Every function returns None, having done nothing, unless each argument is a plain
+// Every function returns None, having written nothing, unless each argument is a plain
 // dense GPU tensor of the type and layout that the chain takes as it is; ops.py then
-// goes the general way, which converts, copies or refuses.  Nothing is kept between
-// calls.  Tensors come from the caching allocator on the current stream, like those
-// of the general way, so the calls can be captured in a graph.
+// goes the general way, which converts, copies or refuses.  The one product that goes
+// through torch's dispatcher (the router's logits) is checked like an argument: a mode
+// such as autocast may have changed its type.  Nothing is kept between calls.  Tensors
+// come from the caching allocator on the current stream, like those of the general
+// way, so the calls can be captured in a graph.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -427,8 +429,11 @@ PyObject* py_moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
             c10::DeviceGuard guard(x.device());
             void* st = stream_of(x);
             const int64_t T = r.M, H = r.K, R = T * k;
+            // a dispatched product: under autocast it comes back in 16 bits, which
+            // the general way refuses
             const Tensor logits = at::linear(x.to(at::kFloat), gate);
-            need(logits.is_contiguous());
+            need(logits.scalar_type() == at::kFloat && logits.is_contiguous() &&
+                 logits.dim() == 2 && logits.size(0) == T && logits.size(1) == E);
             Scratch sc;
             const int64_t topw = sc.take(2 * R), topi = sc.take(4 * R), seg = sc.take(4 * (E + 1)),
                           map = sc.take(4 * R), pos = sc.take(4 * R), xq = sc.take(T * H),

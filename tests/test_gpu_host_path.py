@@ -144,6 +144,24 @@ def test_moe_forms(pkg, cuda, general, G, T, scoring, groups):
     _same(moe(x), want)
 
 
+@pytest.mark.parametrize("G", [0, 64])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_moe_under_autocast_is_refused(pkg, cuda, G, dtype):
+    """Autocast makes the router's product a 16-bit tensor, half the bytes that the
+    routing kernel would read: the native call declines and `moe_route` refuses.  A
+    region with autocast off inside it routes as outside."""
+    H, I, E = 512, 256, 16
+    experts = [(_weight(pkg, 2 * I, H, G, 10 + e), _weight(pkg, H, I, G, 50 + e)) for e in range(E)]
+    moe = pkg.SparseMoE(gate=(torch.randn(E, H) / 16).half().cuda(), experts=experts, top_k=3)
+    x = torch.randn(1, 9, H).half().cuda()
+    want = moe(x)
+    with torch.autocast("cuda", dtype):
+        with pytest.raises(ValueError, match="fp32 logits"):
+            moe(x)
+        with torch.autocast("cuda", enabled=False):
+            _same(moe(x), want)
+
+
 def test_refusals_are_the_general_ways(pkg, cuda):
     qt = _weight(pkg, 64, 128, 0, 7)
     x = torch.randn(2, 128).half().cuda()
