@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libfni8amd.so")
@@ -89,17 +90,27 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+class _General:
+    """The host path where the native one does not load: every call declines (None), so
+    ops.py goes the general way, which needs the C library only."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def host():
-    """The native host path (csrc/host.cpp, built next to the library); RuntimeError if
-    it is not there."""
+    """The native host path (csrc/host.cpp, built next to the library).  Where it does
+    not load, a warning says so once and the general way takes every call."""
     global _host
     if _host is None:
         load()
         try:
             from . import _host as module
         except ImportError as e:
-            raise RuntimeError(f"{os.path.join(_PKG_DIR, '_host.so')} does not load: build it with "
-                               f"`make -C {os.path.join(_PKG_DIR, 'csrc')}`") from e
+            warnings.warn(f"the native host path does not load ({e}); calls take the general way, "
+                          f"with more host time each: `make -C {os.path.join(_PKG_DIR, 'csrc')}` "
+                          "builds it", RuntimeWarning, stacklevel=2)
+            module = _General()
         _host = module
     return _host
 
