@@ -99,13 +99,18 @@ class _General:
 
 
 def host():
-    """The native host path (csrc/host.cpp, built next to the library).  Where it does
-    not load, a warning says so once and the general way takes every call."""
+    """The native host path (csrc/host.cpp, built next to the library for one Python and
+    one torch).  Where it does not load or was built for another torch, a warning says
+    so once and the general way takes every call."""
     global _host
     if _host is None:
         load()
+        import torch
         try:
             from . import _host as module
+            built = getattr(module, "torch_version", None)
+            if built != torch.__version__:
+                raise ImportError(f"built for torch {built}, not {torch.__version__}")
         except ImportError as e:
             warnings.warn(f"the native host path does not load ({e}); calls take the general way, "
                           f"with more host time each: `make -C {os.path.join(_PKG_DIR, 'csrc')}` "

@@ -475,4 +475,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }
+// torch_version: the torch this was compiled against, which _lib.py compares before
+// the first call (torch's C++ ABI holds for one build only).
+PyMODINIT_FUNC PyInit__host(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", FNI8_TORCH_VERSION) < 0) Py_CLEAR(m);
+    return m;
+}

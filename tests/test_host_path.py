@@ -2,10 +2,12 @@
 import os
 import subprocess
 import sys
+import sysconfig
 import warnings
 from importlib import import_module
 
 import pytest
+import torch
 
 
 def test_general_way_where_the_module_does_not_load(pkg, monkeypatch):
@@ -19,6 +21,19 @@ def test_general_way_where_the_module_does_not_load(pkg, monkeypatch):
         for name in ("linear", "gemm", "mlp", "rmsnorm", "moe"):
             assert getattr(lib.host(), name)(None, 1) is None
     assert [w.category for w in seen] == [RuntimeWarning]
+
+
+def test_module_of_another_build_is_not_used(pkg, monkeypatch):
+    """The module is tied to one Python (its file name) and one torch (checked)."""
+    lib = import_module("fni8serve_amd._lib")
+    native = import_module("fni8serve_amd._host")
+    assert native.__file__.endswith("_host" + sysconfig.get_config_var("EXT_SUFFIX"))
+    monkeypatch.setattr(lib, "_host", None)
+    assert lib.host() is native
+    monkeypatch.setattr(lib, "_host", None)
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    with pytest.warns(RuntimeWarning, match="0.0.0"):
+        assert lib.host().linear(None) is None
 
 
 @pytest.mark.parametrize("python,host", [(sys.executable, True), (sys.executable + " -S", False)])
