@@ -17,7 +17,7 @@ from torch.nn.modules.module import _has_any_global_hook
 
 from .. import ops
 from ..qtensor import QTensor
-from .activation import SiluAndMul, fused_act, get_act_and_mul
+from .activation import GeluAndMul, SiluAndMul, fused_act, get_act_and_mul
 from .linear import LinearW8A8
 
 # Rows from which the fused activation + quantization feeds the down projection.
@@ -29,13 +29,27 @@ from .linear import LinearW8A8
 FUSE_MIN_ROWS = 5
 
 
+# What calling one of these modules runs, as their classes were defined.
+_CALL = getattr(nn.Module, "_wrapped_call_impl", None)
+_DEFINED = {cls: [(name, getattr(cls, name)) for name in names]
+            for cls, names in ((LinearW8A8, ("forward", "_int8_ok")),
+                               (SiluAndMul, ("forward",)), (GeluAndMul, ("forward",)))}
+
+
 def bare(m: nn.Module, cls: type) -> bool:
-    """True when calling `m` is calling cls.forward and nothing else: exactly that class,
-    no hook on it or on every module, no forward of its own."""
+    """True when calling `m` is calling the forward that `cls` was defined with and nothing
+    else: exactly that class, no hook on it or on every module, not compiled, and no
+    method of its own or put on the class since."""
     d = m.__dict__
-    return (type(m) is cls and "forward" not in d
-            and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-                     or d["_backward_pre_hooks"] or _has_any_global_hook()))
+    if (type(m) is not cls or cls not in _DEFINED or cls.__call__ is not _CALL
+            or d.get("_compiled_call_impl") is not None
+            or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+            or d["_backward_pre_hooks"] or _has_any_global_hook()):
+        return False
+    for name, defined in _DEFINED[cls]:
+        if name in d or getattr(cls, name) is not defined:
+            return False
+    return True
 
 
 class GatedMLP(nn.Module):

@@ -123,6 +123,32 @@ def test_mlp_module_surgery(pkg, cuda):
     assert not torch.equal(m(x), plain)
 
 
+@pytest.mark.parametrize("M", [2, 9])
+def test_mlp_replaced_steps_run(pkg, cuda, general, monkeypatch, M):
+    """A compiled part, a rule of its own and a forward put on the class run in the MLP as
+    they do the general way."""
+    H, I = 256, 128
+    x = torch.randn(M, H).half().cuda()
+    linear = pkg.LinearW8A8
+
+    def changed(surgery):
+        with monkeypatch.context() as mp:
+            m = pkg.GatedMLP(_weight(pkg, 2 * I, H, 0, 5), _weight(pkg, H, I, 0, 6))
+            before = m(x)
+            surgery(m, mp)
+            with general():
+                want = m(x)
+            _same(m(x), want)
+            return not torch.equal(want, before)
+
+    assert changed(lambda m, mp: mp.setattr(
+        m.gate_up_proj, "_compiled_call_impl", lambda v: 2 * linear.forward(m.gate_up_proj, v)))
+    assert changed(lambda m, mp: mp.setattr(
+        linear, "forward", lambda self, v: 2 * pkg.linear(v, self.weight)))
+    changed(lambda m, mp: mp.setattr(m.gate_up_proj, "_int8_ok", lambda v: False, raising=False))
+    changed(lambda m, mp: mp.setattr(type(m.act_fn), "forward", lambda self, v: v[..., :I] * 0))
+
+
 @pytest.mark.parametrize("G", [0, 64])
 @pytest.mark.parametrize("T", [1, 9, 300])
 @pytest.mark.parametrize("scoring,groups", [("softmax", None), ("sigmoid", 4)])

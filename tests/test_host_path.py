@@ -46,3 +46,32 @@ def test_make_without_torch_builds_the_library(pkg, python, host):
     assert plan.returncode == 0 and plan.stderr == ""
     assert "-shared -o ../libfni8amd.so" in plan.stdout
     assert ("host.cpp" in plan.stdout) == host
+
+
+_SURGERY = {
+    "hook": lambda m, mp: m.register_forward_hook(lambda *a: None),
+    "pre_hook": lambda m, mp: m.register_forward_pre_hook(lambda *a: None),
+    "own_forward": lambda m, mp: mp.setattr(m, "forward", lambda x: x, raising=False),
+    "class_forward": lambda m, mp: mp.setattr(type(m), "forward", lambda self, x: x),
+    "class_call": lambda m, mp: mp.setattr(type(m), "__call__", lambda self, x: x, raising=False),
+    "compiled": lambda m, mp: mp.setattr(m, "_compiled_call_impl", lambda x: x),
+    "subclass": lambda m, mp: setattr(m, "__class__", type("Sub", (type(m),), {})),
+    "own_rule": lambda m, mp: mp.setattr(m, "_int8_ok", lambda x: False, raising=False),
+    "class_rule": lambda m, mp: mp.setattr(type(m), "_int8_ok", lambda self, x: False, raising=False),
+}
+
+
+@pytest.mark.parametrize("surgery", sorted(_SURGERY))
+@pytest.mark.parametrize("part", ["gate_up_proj", "down_proj", "act_fn"])
+def test_bare_sees_module_surgery(pkg, monkeypatch, surgery, part):
+    """The one-call MLP is for untouched parts: whatever else a call would run shows."""
+    bare = import_module("fni8serve_amd.layers.mlp").bare
+    qt = [pkg.QTensor(torch.zeros(n, k, dtype=torch.int8), torch.ones(n), scheme="per_row_i8")
+          for n, k in ((16, 8), (8, 8))]
+    m = getattr(pkg.GatedMLP(*qt), part)
+    cls = type(m)
+    assert bare(m, cls)
+    _SURGERY[surgery](m, monkeypatch)
+    if part == "act_fn" and surgery.endswith("rule"):
+        return  # an activation has no such rule
+    assert not bare(m, cls)
