@@ -66,10 +66,6 @@ def _w4_stackable(qs: list[QTensor]) -> bool:
                for q in qs)
 
 
-# the steps that `_native` does in one call, unless an instance has its own
-_STEPS = ("route", "experts_grouped", "experts_grouped_w4")
-
-
 class SparseMoE(nn.Module):
     def __init__(self, *, gate: torch.Tensor, experts: list[tuple[QTensor, QTensor]], top_k: int,
                  norm_topk_prob: bool = True, act: str = "silu",
@@ -254,7 +250,8 @@ class SparseMoE(nn.Module):
         they have to run one by one."""
         act = fused_act(self.act_fn)
         if (act is None or type(self) is not SparseMoE or not (self.grouped or self.grouped_w4)
-                or not self.__dict__.keys().isdisjoint(_STEPS)):
+                or not self.__dict__.keys().isdisjoint(_STEPS)
+                or any(getattr(SparseMoE, n) is not step for n, step in _STEPS.items())):
             return None
         g1, g2 = (0, 0) if self.grouped else (self.g_gate_up, self.g_down)
         return ops.sparse_moe(xf, self._gate_f32(), self.top_k, self.scoring_func,
@@ -283,3 +280,8 @@ class SparseMoE(nn.Module):
                 shared_out = shared_out * g
             out = out + shared_out
         return out.reshape(B, S, H)
+
+
+# the steps that `_native` does in one call, unless an instance has its own or another
+# one has been put on the class
+_STEPS = {n: getattr(SparseMoE, n) for n in ("route", "experts_grouped", "experts_grouped_w4")}

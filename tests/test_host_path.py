@@ -75,3 +75,19 @@ def test_bare_sees_module_surgery(pkg, monkeypatch, surgery, part):
     if part == "act_fn" and surgery.endswith("rule"):
         return  # an activation has no such rule
     assert not bare(m, cls)
+
+
+@pytest.mark.parametrize("owner", ["instance", "class"])
+@pytest.mark.parametrize("step", ["route", "experts_grouped", "experts_grouped_w4"])
+def test_moe_steps_replaced(pkg, monkeypatch, owner, step):
+    """SparseMoE's one call is for the steps that the class was defined with."""
+    ops = import_module("fni8serve_amd.ops")
+    monkeypatch.setattr(ops, "sparse_moe", lambda *a: "one call")
+    qt = [pkg.QTensor(torch.zeros(n, k, dtype=torch.int8), torch.ones(n), scheme="per_row_i8")
+          for n, k in ((16, 8), (8, 8))]
+    moe = pkg.SparseMoE(gate=torch.zeros(2, 8), experts=[qt, qt], top_k=1)
+    x = torch.zeros(3, 8)
+    assert moe._native(x) == "one call"
+    monkeypatch.setattr(moe if owner == "instance" else pkg.SparseMoE, step, lambda *a: None,
+                        raising=False)
+    assert moe._native(x) is None
