@@ -32,7 +32,7 @@ __global__ __launch_bounds__(WAVES * 64) void moe_sort_kernel(
     const int e = blockIdx.x;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int steps = (Tk + STEP * WAVES - 1) / (STEP * WAVES);
+    const int steps = (Tk - 1) / (STEP * WAVES) + 1;  // rounded up; no sum here passes 2^31
     const int64_t first = (int64_t)wave * steps * STEP + lane * 4;
 
     // ids i .. i+3 (-1 past the end)

@@ -41,3 +41,24 @@ def test_sort_ids_out_of_range(pkg, cuda, T):
     assert np.array_equal(rt.cpu().numpy()[:order.size], order // k)
     assert np.array_equal(seg.cpu().numpy(),
                           np.searchsorted(flat[order], np.arange(E + 1), side="left"))
+
+
+def test_sort_most_ids(pkg, cuda):
+    """The largest T * k that the entry point takes: no count on the way passes 2^31.
+    Three ids of expert 1 among ids of expert 0, looked at where the rows change."""
+    T = 2**31 - 1
+    at = [5, 2**30, T - 2]
+    ids = torch.zeros(T, 1, dtype=torch.int32, device="cuda")
+    for i in at:
+        ids[i] = 1
+    seg, rt, pos = pkg.moe_sort(ids, 2)
+    torch.cuda.synchronize()
+    del ids
+    assert seg.tolist() == [0, T - 3, T]
+    assert rt[:7].tolist() == [0, 1, 2, 3, 4, 6, 7]
+    assert rt[T - 5:].tolist() == [T - 3, T - 1] + at
+    assert pos[:7, 0].tolist() == [0, 1, 2, 3, 4, T - 3, 5]
+    assert pos[2**30 - 1:2**30 + 2, 0].tolist() == [2**30 - 2, T - 2, 2**30 - 1]
+    assert pos[T - 3:, 0].tolist() == [T - 5, T - 1, T - 4]
+    del rt, pos
+    torch.cuda.empty_cache()
