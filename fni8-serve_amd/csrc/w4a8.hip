@@ -623,8 +623,11 @@ __global__ __launch_bounds__(WAVES * 64) void w4a8_mfma_kernel(
 // every sum cost a third instruction to move.
 //
 // The sums are 16 * acc_g, and the running sums hold 16 times the fold's value:
-// fma((float)(16 acc_g), ws, 16 accf) rounds exactly as fma((float)acc_g, ws, accf)
-// scaled by 16, and the epilogue multiplies by 1/16 first.
+// fma((float)(16 acc_g), ws, 16 accf) rounds as fma((float)acc_g, ws, accf) scaled by
+// 16 while neither leaves fp32's normal range, and the epilogue multiplies by 1/16
+// first.  Below that range the scaled sums keep more bits.  Above, from 2^124, they are
+// infinities or NaN to the end: a lane that finds one folds its elements again,
+// unscaled (refold), so that the range is fp32's as in the decode kernels.
 //
 // MI355X, 1500 tokens, us before (folds after all products, accumulation registers, two
 // barriers a step; an 8-wave kernel at G = 256) -> now: G = 128 24576 x 4096 307 -> 243,
@@ -927,6 +930,7 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
         if (has_bias && n < N) bcol[j] = fni8::h2f(bias[n]);
     }
     __syncthreads();
+    float past = 0.0f;  // NaN once a running sum is not finite
     // lane l, register r of block (i, j): row 8*(r/4) + 4*(l/32) + r%4, column l%32
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -940,12 +944,42 @@ __global__ __launch_bounds__(256, 2) void w4a8_tile_kernel(
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
                     float v = accf[i][j][4 * q + r] * 0.0625f;
+                    past = __builtin_fmaf(v, 0.0f, past);
                     v = v * asc[r];
                     if (has_bias) v = v + bcol[j];
                     const int col = wn * 64 + j * 32 + (lane & 31);
                     *reinterpret_cast<uint16_t*>(smem + (row + r) * kTileRow + 2 * col) = fni8::f2h(v);
                 }
         }
+    // refold: the lane's 64 elements as the decode kernels fold them (a weight whose
+    // scales reach 2^100, or one that holds infinities or NaN)
+    if (past != past) {
+#pragma unroll 1
+        for (int t = 0; t < 64; t++) {
+            const int row = wm * 64 + (t >> 5) * 32 + 8 * ((t >> 3) & 3) + 4 * (lane >> 5) + ((t >> 1) & 3);
+            const int col = wn * 64 + (t & 1) * 32 + (lane & 31);
+            if (m0 + row >= mend || n0 + col >= N) continue;
+            const int8_t* xr = xq + (int64_t)src_row(m0 + row) * ldq;
+            const uint8_t* wr = w + (int64_t)(n0 + col) * (K / 2);
+            const float* sr = ws + (int64_t)(n0 + col) * ng;
+            float v = 0.0f;
+#pragma unroll 1
+            for (int g = 0; g < ng; g++) {
+                int acc = 0;
+                for (int k = g * G; k < (g + 1) * G; k += 8) {
+                    const uint2 xv = *reinterpret_cast<const uint2*>(xr + k);
+                    uint32_t xe, xo, ce, co;
+                    split8(xv.x, xv.y, xe, xo);
+                    unpack8(*reinterpret_cast<const uint32_t*>(wr + k / 2), ce, co);
+                    acc = dot4(xo, co, dot4(xe, ce, acc));
+                }
+                v = __builtin_fmaf((float)acc, sr[g], v);
+            }
+            v = v * scl[row];
+            if (has_bias) v = v + fni8::h2f(bias[n0 + col]);
+            *reinterpret_cast<uint16_t*>(smem + row * kTileRow + 2 * col) = fni8::f2h(v);
+        }
+    }
     __syncthreads();
     const int col = n0 + (tid & 15) * 8;
     if (col >= N) return;

@@ -470,3 +470,37 @@ def test_sparse_moe_w4_graph_capture(pkg, T):
             torch.cuda.synchronize()
             assert torch.isfinite(want).all()
             assert torch.equal(y_static, want), rep
+
+
+@pytest.mark.parametrize("G,grouped", [(32, False), (64, False), (128, False), (256, False),
+                                       (64, True), (128, True), (256, True)])
+def test_w4a8_tile_range(pkg, G, grouped):
+    """The tile kernel's sums reach as far as fp32 does: group scales near 2^112 take most
+    of them past 2^124, some past 2^126, and tiny row scales bring the output back; one
+    column holds a NaN scale, one an infinite one.  Bits as the oracle's, NaN where it has
+    NaN."""
+    M, N, K = 65, 200 if grouped else 8200, 512
+    if not grouped:  # more workgroups than the sliced decode kernel takes
+        assert -(-N // 16) * -(-M // 64) > 512
+    rng = np.random.default_rng(G)
+    xq = rng.integers(-127, 128, (M, K)).astype(np.int8)
+    w = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    ws = (rng.uniform(0.5, 1.0, (N, K // G)) * 2.0**112).astype(np.float32)
+    xs = (rng.uniform(0.5, 1.0, M) * 2.0**-118).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float16)
+    ws[3, 1], ws[5, 0] = np.nan, np.inf
+    d = [torch.from_numpy(a).cuda() for a in (xq, xs, w, ws, bias)]
+    if grouped:
+        seg = torch.tensor([0, M], dtype=torch.int32, device="cuda")
+        y = pkg.ops.gemm_w4a8_grouped(d[0], d[1], d[2][None], d[3][None], G, seg, M, bias=d[4][None])
+    else:
+        y = pkg.gemm_quantized(d[0], d[1], pkg.QTensor(d[2], d[3], scheme="per_group_i4",
+                                                       group_size=G, codebook="int4"), d[4])
+    cols = np.unique(np.r_[0:40, N - 40:N])
+    want = o.gemm_w4a8(xq, xs, w[cols], ws[cols], G, bias=bias[cols])
+    got = y.cpu().numpy()[:, cols]
+    nan = np.isnan(want)
+    assert np.isfinite(want[:, 6:]).all() and nan[:, 3].all()
+    assert (np.abs(want.astype(np.float64)) / xs[:, None] > 2.0**126).any()
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan].view(np.uint16), want[~nan].view(np.uint16))
