@@ -278,17 +278,30 @@ int rowblock_grouped_launch(const int8_t* aq, const float* as, const int32_t* rm
     return FNI8_OK;
 }
 
+int cu_count() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            n <= 0)
+            n = 256;
+        return n;
+    }();
+    return cus;
+}
+
 template <int G>
 int grouped_by_tile(const int8_t* aq, const float* as, const int32_t* rmap, int64_t R_max,
                     int64_t K, const uint8_t* w, const float* ws, int64_t E, int64_t N,
-                    const int32_t* seg_off, const uint16_t* bias, uint16_t* y, hipStream_t st) {
-    // Segment tiles of 16 or 32 rows by the mean rows per expert, four
+                    const int32_t* seg_off, const uint16_t* bias, uint16_t* y, bool rows64,
+                    hipStream_t st) {
+    // Segment tiles of 16, 32 or 64 rows by the mean rows per expert, four
     // waves.  Measured on the Qwen3-30B-A3B projections (128 experts, top-8,
     // uniform routing; gate_up [1536, 2048], down [2048, 768]), µs against the
     // earlier 16-row, two-wave, two-slab shape: T = 16 gate_up 30.44 / 32.69,
     // down 18.87 / 21.97 (16-row tiles); T = 256 gate_up 62.61 / 81.28, down
     // 40.41 / 49.11 (32-row tiles).  One slab per batch was faster than two at
-    // every small-segment point.
+    // every small-segment point; 64-row tiles keep two where K allows.
     // With few rows (T = 1: 8 of 128 experts) four-wave workgroups would leave
     // the grid under two per CU; the two-wave shape stays there.
     const double avg = (double)R_max / (double)E;
@@ -302,8 +315,13 @@ int grouped_by_tile(const int8_t* aq, const float* as, const int32_t* rmap, int6
     if (avg <= 8.0)
         return rowblock_grouped_launch<1, 4, 1, G>(aq, as, rmap, R_max, K, w, ws, E, N, seg_off,
                                                    bias, y, st);
-    return rowblock_grouped_launch<2, 4, 1, G>(aq, as, rmap, R_max, K, w, ws, E, N, seg_off, bias,
-                                               y, st);
+    if (!rows64)
+        return rowblock_grouped_launch<2, 4, 1, G>(aq, as, rmap, R_max, K, w, ws, E, N, seg_off,
+                                                   bias, y, st);
+    return sb2 ? rowblock_grouped_launch<4, 4, 2, G>(aq, as, rmap, R_max, K, w, ws, E, N, seg_off,
+                                                     bias, y, st)
+               : rowblock_grouped_launch<4, 4, 1, G>(aq, as, rmap, R_max, K, w, ws, E, N, seg_off,
+                                                     bias, y, st);
 }
 
 }  // namespace
@@ -354,17 +372,36 @@ int launch_gemm_w4a8_grouped(const int8_t* aq, const float* as, const int32_t* r
                              const uint16_t* bias, uint16_t* y, hipStream_t st) {
     if (R_max == 0) return FNI8_OK;
     // More than 32 rows per expert on average: 128x128 segment tiles of the prefill
-    // tile kernel (w4a8.hip).  gate_up + down of 128 experts, hidden 2048, inter 768,
-    // G = 128, us here : there, uniform routing / Zipf-skewed: 24 rows 128 : 147 /
-    // 147 : 137, 32 rows 155 : 148 / 168 : 148, 40 rows 182 : 151 / 226 : 169,
-    // 63 rows 267 : 159 / 290 : 195 (here: 64-row tiles above 32 rows).
-    if (R_max > 32 * E)
+    // tile kernel (w4a8.hip).  gate_up + down of 128 experts, hidden 2048, inter 768, us
+    // here (32-row tiles; above 32 rows 64-row ones) : there, uniform routing /
+    // Zipf-skewed: G = 128 24 rows 120 : 141 / 136 : 159, 32 rows 147 : 148 / 157 : 165,
+    // 33 rows 157 : 150 / 182 : 170, 63 rows 250 : 158 / 261 : 187; G = 64 32 rows
+    // 154 : 163 / 167 : 186, 33 rows 184 : 165 / 214 : 191; G = 256 32 rows 139 : 131 /
+    // 148 : 149, 33 rows 149 : 139 / 171 : 153.
+    //
+    // Below 64 rows the tile kernel has one row tile an expert or little more.  Where
+    // those leave CUs idle, the row-block kernel's 64-row workgroups fill more of them:
+    // 64-row tiles (fewer reads of the weights) up to 40 rows from K = 1024, and up to 63
+    // from K = 2048 on at most half of the CUs; else 32-row tiles.  Time as a share of the tile
+    // kernel's at 33 / 40 / 50 / 63 rows, G = 128, uniform routing, 64-row | 32-row
+    // tiles, by (experts, N, K): (4, 2048, 4096) .61 .62 .66 .68 | .82 .83 .82 .83;
+    // (16, 1024, 2048) .78 .77 .83 .92 | .84 .90 .88 .96; (16, 1536, 2048) .78 .79 .75
+    // 1.14 | .85 .97 .81 .94; (16, 1024, 768) 1.01 1.03 1.12 1.17 | .92 1.01 1.00 1.03.
+    // As many workgroups as CUs, (16, 2048, 2048): .95 1.01 1.11 1.37 | .77 .93 .93 1.37;
+    // only long K gains on 64-row tiles there, (8, 4096, 14336): .72 .72 .79 .95.
+    const double avg = (double)R_max / (double)E;
+    const int64_t tiles = E * ((N + 127) / 128);
+    const int cus = cu_count();
+    const bool rows64 = avg > 32.0 && ((tiles < cus && K >= 1024 && avg <= 40.0) ||
+                                       (2 * tiles <= cus && K >= 2048) ||
+                                       (tiles <= cus && K >= 8192 && avg <= 48.0));
+    if (avg >= 64.0 || (avg > 32.0 && tiles >= cus && !rows64))
         return launch_w4a8_tile_grouped(aq, as, row_index, R_max, K, w, ws, E, N, G, seg_off,
                                         bias, y, st);
     switch (G) {
-        case 64: return grouped_by_tile<64>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, st);
-        case 128: return grouped_by_tile<128>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, st);
-        default: return grouped_by_tile<256>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, st);
+        case 64: return grouped_by_tile<64>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, rows64, st);
+        case 128: return grouped_by_tile<128>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, rows64, st);
+        default: return grouped_by_tile<256>(aq, as, row_index, R_max, K, w, ws, E, N, seg_off, bias, y, rows64, st);
     }
 }
 

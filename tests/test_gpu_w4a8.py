@@ -398,7 +398,7 @@ def test_w4a8_grouped_gemm_bitexact(pkg, per_expert, E, N, K, G):
     """The grouped W4A8 GEMM against the oracle expert by expert: ragged
     segments (one expert empty), the row-block kernel's 16-row segment tiles
     on two waves (mean 1 row per expert, a small grid) and on four (mean 4, 64
-    experts), its 32- and 64-row tiles (20, 60) and the tile kernel's 128-row
+    experts), its 32-row tiles (20, 60) and the tile kernel's 128-row
     ones (150), K = 768 (odd slab count) and 1024, activation rows gathered
     through a row map, bias, and `rows` beyond the sorted rows (those are not
     written)."""
@@ -504,3 +504,33 @@ def test_w4a8_tile_range(pkg, G, grouped):
     assert (np.abs(want.astype(np.float64)) / xs[:, None] > 2.0**126).any()
     assert np.array_equal(np.isnan(got), nan)
     assert np.array_equal(got[~nan].view(np.uint16), want[~nan].view(np.uint16))
+
+
+@pytest.mark.parametrize("G", [64, 128, 256])
+@pytest.mark.parametrize("mean,E,N,K", [(32, 4, 200, 1024), (33, 4, 200, 1024), (40, 4, 200, 1280),
+                                        (41, 4, 200, 1024), (33, 4, 200, 768), (63, 4, 200, 2304),
+                                        (63, 4, 200, 2048), (64, 4, 200, 2048),
+                                        (41, 2, 8200, 2048), (63, 2, 16256, 768),
+                                        (33, 2, 16384, 1024), (48, 2, 16384, 8192),
+                                        (49, 2, 16384, 8192)])
+def test_w4a8_grouped_rule_edges(pkg, mean, E, N, K, G):
+    """The choice of segment tiles between 32 and 64 mean rows per expert, at its lines:
+    32 | 33 and 40 | 41 and 63 | 64 rows, K from 1024 and from 2048 with an odd and an
+    even number of slabs and long K up to 48 rows (64-row tiles), 130 column tiles (more than half of the CUs: 32
+    rows), 254 and 256 (the tile kernel).  Ragged segments, sampled columns, bit for bit."""
+    rng = np.random.default_rng(mean + N + K + G)
+    lens = rng.multinomial(mean * E, np.ones(E) / E)
+    seg = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    R = int(seg[-1])
+    xq = rng.integers(-127, 128, (R, K)).astype(np.int8)
+    xs = rng.uniform(0.001, 0.05, R).astype(np.float32)
+    w = rng.integers(0, 256, (E, N, K // 2), dtype=np.uint8)
+    ws = rng.uniform(1e-3, 2e-2, (E, N, K // G)).astype(np.float32)
+    y = pkg.ops.gemm_w4a8_grouped(*(torch.from_numpy(a).cuda() for a in (xq, xs, w, ws)), G,
+                                  torch.from_numpy(seg).cuda(), R)
+    cols = np.unique(np.r_[0:17, N - 17:N, rng.integers(0, N, 30)])
+    got = y.cpu().numpy()[:, cols]
+    for e in range(E):
+        lo, hi = seg[e], seg[e + 1]
+        want = o.gemm_w4a8(xq[lo:hi], xs[lo:hi], w[e][cols], ws[e][cols], G)
+        assert np.array_equal(got[lo:hi].view(np.uint16), want.view(np.uint16)), e
