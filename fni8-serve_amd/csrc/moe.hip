@@ -6,7 +6,7 @@
 //          global atomics.  Pass 2 places the wave's entries in id order (the
 //          rank inside 256 ids from four ballots), so the segment keeps the
 //          (token, slot) order of `(topi == e).nonzero()` -- a deterministic,
-//          stable counting sort.  Up to 2048 ids a wave stay in registers
+//          stable counting sort.  Up to 1024 ids a wave stay in registers
 //          between the passes.
 // combine: one workgroup per token; each lane owns 8 consecutive hidden
 //          elements and sums the token's expert rows in ascending expert id
@@ -19,15 +19,15 @@ namespace {
 constexpr int kMaxTopK = 32;
 
 // Bound by latency: every workgroup reads all ids (from L2) and meets once.
-// Walking 1024 ids at a time with two block barriers each took 47 us for 24000
-// ids and 128 experts on MI355X; this takes 9 (16 waves; few ids keep 4 waves,
-// which start sooner).
-template <int WAVES>
+// Walking 1024 ids at a time with two block barriers each took 48 us for 24000
+// ids and 128 experts on MI355X; this takes 8.3 (16 waves).
+// KEEP: steps held in registers; each costs its share of the start, so as few as
+// the ids of a launch need.
+template <int WAVES, int KEEP>
 __global__ __launch_bounds__(WAVES * 64) void moe_sort_kernel(
     const int32_t* __restrict__ topi, int Tk, int k, int E, int32_t* __restrict__ seg_off,
     int32_t* __restrict__ row_token, int32_t* __restrict__ pos) {
     constexpr int STEP = 256;  // ids per wave and step, four per lane
-    constexpr int KEEP = 8;    // steps held in registers
     __shared__ int lds[2][WAVES];
     const int e = blockIdx.x;
     const int lane = threadIdx.x & 63;
@@ -256,13 +256,18 @@ namespace fni8h {
 
 int launch_moe_sort(const int32_t* topi, int64_t T, int64_t k, int64_t E, int32_t* seg_off,
                     int32_t* row_token, int32_t* pos, hipStream_t st) {
-    // 4 waves hold 2048 ids in two steps each; above, 16 waves
-    if (T * k <= 2048)
-        hipLaunchKernelGGL(moe_sort_kernel<4>, dim3((unsigned)E), dim3(4 * 64), 0, st, topi,
-                           (int)(T * k), (int)k, (int)E, seg_off, row_token, pos);
-    else
-        hipLaunchKernelGGL(moe_sort_kernel<16>, dim3((unsigned)E), dim3(16 * 64), 0, st, topi,
-                           (int)(T * k), (int)k, (int)E, seg_off, row_token, pos);
+    // us on MI355X by (ids, experts), 4 waves and 2 steps : 8 and 4 : 16 and 4 (and before,
+    // walking 1024 ids at a time): (16, 128) 2.6 : 3.0 : 3.6 (3.3), (2048, 128) 3.3 :
+    // 3.3 : 3.8 (6.0), (24000, 128) 18.8 : 11.3 : 8.3 (48.1).  More than one workgroup a
+    // CU: (16, 512) 2.7 : 3.4 : 5.6 (3.4), (3000, 512) 4.0 : 4.1 : 6.0 (7.7), (24000, 512)
+    // 16.5 : 10.9 : 11.5 (47.1).
+#define FNI8_SORT(WAVES, KEEP)                                                                  \
+    hipLaunchKernelGGL((moe_sort_kernel<WAVES, KEEP>), dim3((unsigned)E), dim3(WAVES * 64), 0, st, \
+                       topi, (int)(T * k), (int)k, (int)E, seg_off, row_token, pos)
+    if (T * k <= 2048) FNI8_SORT(4, 2);
+    else if (E <= 256) FNI8_SORT(16, 4);
+    else FNI8_SORT(8, 4);
+#undef FNI8_SORT
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error_detail("moe_sort launch: %s", hipGetErrorString(e));

@@ -1,6 +1,7 @@
-"""The routing sort at the edges of its wave and register shares: 2048 ids (4 or
-16 waves), 32768 ids (kept in registers or read again), ragged ends, an id array
-that is only 4-byte aligned, and ids outside [0, E).  Whole numbers: exact."""
+"""The routing sort at the edges of its wave and register shares: 2048 ids (4 or more
+waves), 256 experts (16 or 8 waves), 16384 or 8192 ids (kept in registers or read again),
+ragged ends, an id array that is only 4-byte aligned, and ids outside [0, E).  Whole
+numbers: exact."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +12,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,k,E", [(1, 1, 1), (2047, 1, 7), (2048, 1, 5), (2049, 1, 5), (683, 3, 16),
-                                   (5461, 6, 64), (32768, 1, 3), (32769, 1, 3), (20011, 2, 130)])
+                                   (5461, 6, 64), (32768, 1, 3), (32769, 1, 3), (20011, 2, 130),
+                                   (16384, 1, 256), (16385, 1, 256), (2048, 1, 257),
+                                   (2049, 1, 257), (4096, 2, 300), (8193, 1, 300), (3000, 8, 512)])
 def test_sort_edges(pkg, cuda, T, k, E):
     rng = np.random.default_rng(T + E)
     ids = rng.integers(0, E, size=(T + 1, k)).astype(np.int32)
