@@ -34,6 +34,12 @@ ROUTE_CASES = [
     dict(T=200, E=40, k=12, scoring="softmax", ties=True),
     dict(T=64, E=96, k=4, scoring="sigmoid", nan=True),
     dict(T=64, E=96, k=4, scoring="softmax", nan=True),
+    # eight and more experts a lane, the last ones absent; ties within and across lanes
+    dict(T=40, E=449, k=32, scoring="softmax", ties=True),
+    dict(T=40, E=512, k=8, scoring="sigmoid", ties=True),
+    dict(T=40, E=513, k=32, scoring="sigmoid", bias=True, nan=True),
+    dict(T=40, E=1000, k=12, scoring="softmax", ties=True, groups=8, topk_group=1),
+    dict(T=40, E=1024, k=32, scoring="softmax", nan=True, renorm=False),
 ]
 
 
