@@ -538,10 +538,14 @@ bool act_quant_vec_launch(int ch, const uint16_t* x, int64_t ldx, int64_t M, int
 
 // Rows per launch below which a row gets a 1024-thread workgroup.
 constexpr int64_t kFewRows = 256;
-// Longest row (elements) that one wave takes when there are that many rows: four
-// 8-byte chunks a lane; a 256-thread workgroup has a 16-byte chunk for at least half
-// of its lanes from here on.
-constexpr int64_t kWaveRow = 1024;
+// One wave a row (up to four 8-byte chunks a lane), or a 256-thread workgroup: the wave's
+// longer chain per lane pays where the workgroup leaves most of its lanes without a
+// 16-byte chunk, or the rows are many.  Time as a share of the workgroup's on MI355X, silu,
+// by row length at 256 / 1024 / 1536 / 3072 / 16384 rows: 256 .80 .81 .74 .61 .47; 512
+// .99 .96 .91 .81 .72; 768 1.15 1.08 .95 .81 .71; 1024 1.29 1.26 1.07 .92 .85.
+bool wave_per_row(int64_t M, int64_t I) {
+    return M >= (I <= 512 ? kFewRows : I <= 768 ? 1536 : I <= 1024 ? 3072 : INT64_MAX);
+}
 // Rows per launch up to which, given a workspace, G workgroups share a row
 // (G = the row's 16-byte chunks over 256 threads x kSplitChunks, 2..8).
 constexpr int64_t kSplitRows = 128;
@@ -570,7 +574,7 @@ int act_quant_launch(const uint16_t* x, int64_t ldx, int64_t M, int64_t I, int8_
                            dim3(kThreads), 0, st, x, ldx, (int)M, (int)I, G, q, ldq, s, work,
                            fni8h::xcd_wait_ticks());
         done = true;
-    } else if (vec && M >= kFewRows && I <= kWaveRow) {
+    } else if (vec && wave_per_row(M, I)) {
         const dim3 grid((unsigned)((M + 3) / 4)), block(kThreads);
 #define FNI8_ACTW(CH)                                                                          \
     hipLaunchKernelGGL((act_quant_wave_kernel<ACT, CH>), grid, block, 0, st, x, ldx, (int)M, \

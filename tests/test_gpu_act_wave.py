@@ -1,6 +1,7 @@
-"""act_and_mul_quant with one wave per row: 256 rows and more of up to 1024 elements,
-at the edges of the lanes' 8-byte chunks, with a ragged last workgroup and rows of
-zeros, NaN and infinities; int8 rows and scales bit for bit against the oracle."""
+"""act_and_mul_quant with one wave per row: 256 rows and more of up to 512 elements, 1536
+of up to 768 and 3072 of up to 1024, at the edges of these and of the lanes' 8-byte
+chunks, with a ragged last workgroup and rows of zeros, NaN and infinities; int8 rows and
+scales bit for bit against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -12,7 +13,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
 @pytest.mark.parametrize("M,I", [(256, 8), (257, 248), (258, 256), (259, 264), (256, 512),
-                                 (300, 768), (257, 1024), (256, 1032), (255, 768)])
+                                 (300, 768), (257, 1024), (256, 1032), (255, 768),
+                                 (1535, 512), (1536, 520), (1537, 768), (1536, 776), (3071, 1024),
+                                 (3072, 776), (3073, 1024), (3072, 1032)])
 def test_act_quant_wave_rows(pkg, act, M, I):
     rng = np.random.default_rng(M + I)
     x = (rng.standard_normal((M, 2 * I)) * 4).astype(np.float16)
