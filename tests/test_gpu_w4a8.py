@@ -1,7 +1,7 @@
 """GPU parity of the W4A8 linear (per_group_i4 int4 weights) against the oracle
 (oracle/w4a8_oracle.c): int8 activations, fp32 scales and fp16 outputs bit for
-bit, on the decode GEMVs (1-4 tokens), the MFMA decode kernel (5-64 tokens)
-and the MFMA tile kernel (more tokens), every supported group size, Qwen3-8B's
+bit, on the decode GEMVs (1-4 tokens), the MFMA decode kernel (5-64 tokens, more
+in slices on narrow weights) and the MFMA tile kernel (more tokens), every supported group size, Qwen3-8B's
 shapes and ragged ones.  Each output
 element depends only on its own activation row and weight row, so at full size
 the oracle checks sampled rows and columns.  Also the reference's own W4 seam
@@ -302,13 +302,31 @@ def test_w4a8_mfma_decode_narrow_n(pkg, M, N):
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 264, 1024), (300, 520, 2048), (512, 1000, 4096)])
-def test_w4a8_tile8_group256_bitexact(pkg, M, N, K):
-    """Group size 256 above 64 tokens: the 8-wave two-stage tile kernel (two
-    workgroup rows, ragged M and N, bias), every element against the oracle."""
-    print(f"w4a8 tile8 M={M} N={N} K={K}", flush=True)
+def test_w4a8_slices_group256_bitexact(pkg, M, N, K):
+    """Group size 256 above 64 tokens on narrow weights: slices of the decode kernel
+    (ragged M and N, bias), every element against the oracle."""
+    print(f"w4a8 slices M={M} N={N} K={K}", flush=True)
     qt = _w4(pkg, N, K, 256, seed=M + N)
     bias = torch.randn(N, device="cuda").half()
     _check(pkg, _x(M, K, seed=M * 7 + K), qt, bias)
+
+
+@pytest.mark.parametrize("M,N,K,G", [(130, 4200, 1024, 32), (131, 4200, 1056, 32),
+                                     (130, 4200, 512, 64), (300, 4200, 1024, 64),
+                                     (130, 8200, 1088, 64), (65, 8200, 1024, 128),
+                                     (300, 4200, 1536, 128), (65, 8200, 1024, 256),
+                                     (300, 4200, 2048, 256)])
+def test_w4a8_tile_bitexact(pkg, M, N, K, G):
+    """The dense tile kernel's forms over several steps, beyond what the sliced decode
+    kernel takes (more than two workgroups of 16 weight rows a CU): two groups a step (G =
+    32 and 64), one (K a multiple of G only; G = 128) and half of one (G = 256), ragged M
+    and N, bias; all rows, sampled columns with the last 128 against the oracle."""
+    print(f"w4a8 tile M={M} N={N} K={K} G={G}", flush=True)
+    assert G == 32 or K % 256 != 0 or -(-N // 16) * -(-M // 64) > 512
+    qt = _w4(pkg, N, K, G, seed=M + N)
+    cols = np.r_[np.sort(np.random.default_rng(K).choice(N - 128, 128, replace=False)),
+                 np.arange(N - 128, N)]
+    _check(pkg, _x(M, K, seed=M * 7 + K), qt, torch.randn(N, device="cuda").half(), cols=cols)
 
 
 @pytest.mark.parametrize("T,G,H,I", [(3, 64, 512, 256), (40, 64, 512, 256),
@@ -320,7 +338,7 @@ def test_sparse_moe_w4_experts_against_oracle(pkg, T, G, H, I):
     per_group_i4 for weight_bits=4, convert.py:130-131): the layer output bit for
     bit against the oracle's sort, per-expert W4A8 chain (gate_up, silu-and-mul,
     down) and combine, on the same routing.  G = 64..256 run the grouped
-    W4A8 GEMM (16-row segment tiles at T = 3 and 40, 64-row ones at T = 200,
+    W4A8 GEMM (16-row segment tiles at T = 3 and 40, 32-row ones at T = 200,
     where down's K = 768 is an odd number of slabs, the tile kernel's 128-row
     ones at T = 512); G = 32 keeps the per-expert modules."""
     print(f"w4 moe T={T} G={G}", flush=True)
