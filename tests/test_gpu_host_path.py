@@ -29,6 +29,34 @@ def general(pkg):
     return ctx
 
 
+@pytest.fixture
+def taken(pkg):
+    """taken(f): the native calls that f() makes, as (name, whether it took the call)."""
+    from importlib import import_module
+    lib = import_module("fni8serve_amd._lib")
+    native = lib.host()
+
+    class Recorder:
+        def __init__(self):
+            self.calls = []
+
+        def __getattr__(self, name):
+            def call(*a):
+                out = getattr(native, name)(*a)
+                self.calls.append((name, out is not None))
+                return out
+            return call
+
+    def run(f):
+        lib._host = Recorder()
+        try:
+            f()
+            return lib._host.calls
+        finally:
+            lib._host = native
+    return run
+
+
 def _same(a, b):
     a, b = (t if isinstance(t, (tuple, list)) else (t,) for t in (a, b))
     assert len(a) == len(b)
@@ -61,6 +89,56 @@ def _inputs(K):
     yield x[:, :1].expand(70, 2, K)
     yield torch.as_strided(x, (3, K), (8, 1))  # overlapping rows
     yield x[:0, 0]               # no rows
+
+
+# whether the native path takes each of _inputs
+_TAKEN = [True] * 11 + [False] * 4
+
+
+@pytest.mark.parametrize("G", [0, 64])
+def test_forms_taken(pkg, cuda, taken, G):
+    """The forms that the native path is there for go through it, and the others do not:
+    without this, tests that compare it with the general way would pass if it declined
+    everything."""
+    K = 512
+    qt, w = _weight(pkg, 64, K, G, 1), torch.randn(K).half().cuda()
+    bias = torch.randn(64).half().cuda()
+    m = pkg.GatedMLP(_weight(pkg, 2 * 256, K, G, 3), _weight(pkg, K, 256, G, 4))
+    xs = list(_inputs(K))
+    assert len(xs) == len(_TAKEN)
+    for x, take in zip(xs, _TAKEN):
+        assert taken(lambda: pkg.linear(x, qt)) == [("linear", take)]
+        assert taken(lambda: pkg.linear(x, qt, bias)) == [("linear", take)]
+        assert taken(lambda: pkg.rmsnorm(x, w)) == [("rmsnorm", take)]
+        assert taken(lambda: pkg.rmsnorm_quant(x, w)) == [("rmsnorm", take)]
+        assert taken(lambda: m(x))[:1] == [("mlp", take)]
+        res = x.contiguous()
+        assert taken(lambda: pkg.rmsnorm(x, w, residual=res)) == [("rmsnorm", take)]
+        xq, s = pkg.quantize_rowwise(x)
+        assert taken(lambda: pkg.gemm_quantized(xq, s, qt)) == [("gemm", x.numel() > 0)]
+    x = xs[2]
+    assert taken(lambda: pkg.linear(x, qt, torch.stack([bias, bias], 1)[:, 0])) == [("linear", False)]
+    assert taken(lambda: pkg.rmsnorm(x, w, residual=xs[8][:x.shape[0]])) == [("rmsnorm", False)]
+    graph = torch.cuda.CUDAGraph()
+    m(x)
+
+    def capture():
+        with torch.cuda.graph(graph):
+            m(x)
+    assert taken(capture) == [("mlp", True)]
+
+
+@pytest.mark.parametrize("G", [0, 64])
+def test_moe_taken(pkg, cuda, taken, G):
+    H, I, E = 512, 256, 16
+    experts = [(_weight(pkg, 2 * I, H, G, 10 + e), _weight(pkg, H, I, G, 50 + e)) for e in range(E)]
+    for scoring, kw in (("softmax", {}), ("sigmoid", {"num_expert_groups": 4, "topk_group": 2})):
+        moe = pkg.SparseMoE(gate=(torch.randn(E, H) / 16).half().cuda(), experts=experts, top_k=3,
+                            scoring_func=scoring, **kw)
+        for T in (1, 9, 300):
+            x = torch.randn(1, T, H).half().cuda()
+            assert taken(lambda: moe(x)) == [("moe", True)]
+            assert taken(lambda: moe(torch.cat([x, x], 2)[..., :H])) == [("moe", T == 1)]
 
 
 @pytest.mark.parametrize("G", [0, 32, 128])
