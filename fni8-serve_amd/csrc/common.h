@@ -123,7 +123,10 @@ __device__ __forceinline__ int sum8(int v) {
     return v;
 }
 
-// Max over the wave of non-negative values, returned as a wave-uniform value.
+// Max over the wave of 32-bit values compared as signed ones, returned as a wave-uniform
+// value.  Every lane takes part and no lane's value is replaced by a neutral one, so
+// negative values are as good as others: the router passes keys with the top bit
+// flipped, most of them negative.
 __device__ __forceinline__ uint32_t wave_max_uniform(uint32_t v) {
     int t = (int)v;
     int o;
