@@ -29,27 +29,24 @@ from .linear import LinearW8A8
 FUSE_MIN_ROWS = 5
 
 
-# What calling one of these modules runs, as their classes were defined.
+# What calling one of these modules runs, as their classes were defined: forward and, in
+# a linear, the rule that it asks.
 _CALL = getattr(nn.Module, "_wrapped_call_impl", None)
-_DEFINED = {cls: [(name, getattr(cls, name)) for name in names]
-            for cls, names in ((LinearW8A8, ("forward", "_int8_ok")),
-                               (SiluAndMul, ("forward",)), (GeluAndMul, ("forward",)))}
+_DEFINED = {cls: (cls.forward, getattr(cls, "_int8_ok", None))
+            for cls in (LinearW8A8, SiluAndMul, GeluAndMul)}
 
 
 def bare(m: nn.Module, cls: type) -> bool:
     """True when calling `m` is calling the forward that `cls` was defined with and nothing
-    else: exactly that class, no hook on it or on every module, not compiled, and no
-    method of its own or put on the class since."""
+    else, but for hooks on every module: exactly that class, no hook on it, not compiled,
+    and no method of its own or put on the class since."""
     d = m.__dict__
-    if (type(m) is not cls or cls not in _DEFINED or cls.__call__ is not _CALL
-            or d.get("_compiled_call_impl") is not None
-            or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-            or d["_backward_pre_hooks"] or _has_any_global_hook()):
-        return False
-    for name, defined in _DEFINED[cls]:
-        if name in d or getattr(cls, name) is not defined:
-            return False
-    return True
+    forward, rule = _DEFINED.get(cls, (None, None))
+    return (type(m) is cls and cls.forward is forward and cls.__call__ is _CALL
+            and "forward" not in d and "_compiled_call_impl" not in d
+            and (rule is None or (cls._int8_ok is rule and "_int8_ok" not in d))
+            and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                     or d["_backward_pre_hooks"]))
 
 
 class GatedMLP(nn.Module):
@@ -63,21 +60,22 @@ class GatedMLP(nn.Module):
         self.intermediate_size = self.gate_up_proj.out_features // 2
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        act = fused_act(self.act_fn)
-        if (act is not None and x.is_cuda and bare(self.gate_up_proj, LinearW8A8)
-                and bare(self.down_proj, LinearW8A8) and bare(self.act_fn, type(self.act_fn))):
-            y = ops.gated_mlp(x, self.gate_up_proj.weight, self.down_proj.weight, act,
-                              self.gate_up_proj.bias, self.down_proj.bias, FUSE_MIN_ROWS)
+        gate_up, down, act_fn = self.gate_up_proj, self.down_proj, self.act_fn
+        act = fused_act(act_fn)
+        if (act is not None and x.is_cuda and not _has_any_global_hook()
+                and bare(gate_up, LinearW8A8) and bare(down, LinearW8A8)
+                and bare(act_fn, type(act_fn))):
+            y = ops.gated_mlp(x, gate_up.weight, down.weight, act, gate_up.bias, down.bias,
+                              FUSE_MIN_ROWS)
             if y is not None:
                 return y
         rows = x.numel() // max(x.shape[-1], 1)
-        if (act is not None and rows >= FUSE_MIN_ROWS and self.gate_up_proj._int8_ok(x)
-                and self.down_proj._int8_ok(x)):
-            h = self.gate_up_proj(x)
+        if act is not None and rows >= FUSE_MIN_ROWS and gate_up._int8_ok(x) and down._int8_ok(x):
+            h = gate_up(x)
             xq, xs = ops.act_and_mul_quant(h, act)
-            y = ops.gemm_quantized(xq, xs, self.down_proj.weight, self.down_proj.bias)
+            y = ops.gemm_quantized(xq, xs, down.weight, down.bias)
             return y.reshape(*x.shape[:-1], y.shape[-1])
-        return self.down_proj(self.act_fn(self.gate_up_proj(x)))
+        return down(act_fn(gate_up(x)))
 
 
 class Qwen3MLP(GatedMLP):

@@ -251,7 +251,8 @@ class SparseMoE(nn.Module):
         act = fused_act(self.act_fn)
         if (act is None or type(self) is not SparseMoE or not (self.grouped or self.grouped_w4)
                 or not self.__dict__.keys().isdisjoint(_STEPS)
-                or any(getattr(SparseMoE, n) is not step for n, step in _STEPS.items())):
+                or (SparseMoE.route, SparseMoE.experts_grouped,
+                    SparseMoE.experts_grouped_w4) != _DEFINED):
             return None
         g1, g2 = (0, 0) if self.grouped else (self.g_gate_up, self.g_down)
         return ops.sparse_moe(xf, self._gate_f32(), self.top_k, self.scoring_func,
@@ -284,4 +285,5 @@ class SparseMoE(nn.Module):
 
 # the steps that `_native` does in one call, unless an instance has its own or another
 # one has been put on the class
-_STEPS = {n: getattr(SparseMoE, n) for n in ("route", "experts_grouped", "experts_grouped_w4")}
+_STEPS = ("route", "experts_grouped", "experts_grouped_w4")
+_DEFINED = tuple(getattr(SparseMoE, n) for n in _STEPS)
