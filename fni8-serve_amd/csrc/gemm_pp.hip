@@ -399,8 +399,8 @@ int cu_count() {
 }
 
 // ---- tile and split-K choice ---------------------------------------------------
-// Tiles: {256x256, 256x192, 128x256, 256x128}, and 64x128 for long K at
-// M <= 256 (below); each tile's time per k-tile
+// Tiles: {256x256, 256x192, 128x256, 256x128}, and 64x128 for few rows by rules of
+// its own (the first ones of pp_plan); each tile's time per k-tile
 // relative to 256x256, measured on MI355X over the Qwen3-8B prefill GEMMs:
 // 256x192 takes 0.79 of it for 0.75 of the products (the 2x2 wave arrangement
 // reads 5 fragments per 6 MFMAs instead of 6 per 8), the half-size tiles about
@@ -425,8 +425,10 @@ struct PpPlan {
 
 constexpr double kPartCost = 1.0;     // per 256x256 partial tile merged, in 256x256 k-tiles
 constexpr double kHandoffCost = 1.0;  // counter and last store latency, same unit
-// k-tiles per split at least: with 16 (K = 4096 split in 2) every split plan
-// measured slower than the best unsplit one on Qwen3-8B's shapes at M = 256..2048
+// k-tiles per split at least, for the tiles of 128 and 256 rows: with 16 (K = 4096
+// split in 2) every such plan measured slower than the best unsplit one on Qwen3-8B's
+// shapes at M = 256..2048.  The 64x128 rules take splits from 6 k-tiles on, where
+// their workgroups would not fill the CUs otherwise.
 constexpr int kMinSplitKt = 24;
 
 int g_force_bm = 0, g_force_bn = 0, g_force_split = 0;

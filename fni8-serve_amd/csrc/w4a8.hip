@@ -632,8 +632,9 @@ __global__ __launch_bounds__(WAVES * 64) void w4a8_mfma_kernel(
 // MI355X, 1500 tokens, us before (folds after all products, accumulation registers, two
 // barriers a step; an 8-wave kernel at G = 256) -> now: G = 128 24576 x 4096 307 -> 243,
 // 4096 x 12288 159 -> 140; G = 64 24576 x 4096 405 -> 269; G = 256 24576 x 4096 362 ->
-// 204.  Copies with a part removed (250 whole): without folds 221, without MFMAs 195,
-// without global loads 208, without loads, unpacking and LDS stores 162.
+// 204.  Copies with a part removed, where the whole (243 above) took 250: without folds
+// 221, without MFMAs 195, without global loads 208, without loads, unpacking and LDS
+// stores 162.
 //
 // GROUPED: the expert-segment form (the MoE layer's projections, one launch):
 // blockIdx.x is one 128-row tile of one expert's sorted segment, blockIdx.y the
